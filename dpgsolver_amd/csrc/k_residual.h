@@ -18,9 +18,9 @@
 //   metrics    [E][d*d][Nc]              (metrics_vc (Nc, d, d))
 //   nJ         [F][Nfc][d]               (normals_fc * jacobian_det_fc, left element)
 //   elem faces [E][2d] {f, en, lfN | side<<4 | ord<<8 | bc<<12}
-// Work mapping: one thread per volume node, EPB elements per workgroup, 1-D operators
-// and face orientation tables in LDS, pencil sweeps through LDS (a thread owns one
-// N-long line, reads it to registers, writes its N outputs).
+// Work mapping: one thread per volume node, EPB elements per workgroup, 1-D operators in
+// scalar registers, face orientation tables in LDS, pencil sweeps through LDS (a thread
+// owns one N-long line, reads it to registers, writes its N outputs).
 #pragma once
 
 #include "dgx_device.h"
