@@ -1455,10 +1455,7 @@ dgx_status dgx_assemble_diag_blocks(dgx_ctx* h, const double* u, const double* m
 	Ctx& c = h->c;
 	if (!c.mesh_ready) return c.hp ? DGX_ERR_UNSUPPORTED : DGX_ERR_NO_MESH;
 	if (c.d != 2 && c.d != 3) return DGX_ERR_UNSUPPORTED;   // 3-D: Euler and advection
-	const int nb = c.Np * c.nv;
-	for (int col = 0; col < nb; ++col) DGX_TRY(dgx::launch_diag_col(c, u, blocks, col));
-	if (mass_scale) DGX_TRY(dgx::launch_sub_mass(c, blocks, mass_scale, 0.0));
-	return DGX_OK;
+	return hip_status(dgx::launch_diag_blocks(c, u, mass_scale, blocks));
 }
 
 dgx_status dgx_assemble_face_blocks(dgx_ctx* h, const double* u, double* blocks)
@@ -1477,8 +1474,7 @@ dgx_status dgx_assemble_face_blocks(dgx_ctx* h, const double* u, double* blocks)
 	const int nfv = c.nv * (c.d == 2 ? c.N : c.N * c.N);   // face-node rows / columns of a face block
 	double* cT = nullptr;
 	DGX_TRY(hipMalloc(&cT, sizeof(double) * (size_t)c.E * 2 * c.d * nfv * nfv));
-	hipError_t e = hipSuccess;
-	for (int col = 0; col < nfv && e == hipSuccess; ++col) e = dgx::launch_offd_col(c, u, cT, col);
+	hipError_t e = dgx::launch_offd_blocks(c, u, cT);
 	if (e == hipSuccess) e = dgx::launch_expand_face_blocks(c, cT, blocks);
 	const hipError_t es = hipStreamSynchronize(c.stream);
 	(void)hipFree(cT);

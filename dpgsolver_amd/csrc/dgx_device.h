@@ -112,6 +112,16 @@ template <typename T> struct RealOf { using type = T; };
 template <> struct RealOf<Dual> { using type = double; };
 template <> struct RealOf<Dual32> { using type = double; };   // FP64 vectors in and out
 
+// A pointer to memory that no kernel writes, in the constant address space: loads with uniform indices are then scalar
+// loads also behind the kernel's own stores.
+template <typename T>
+using ConstPtr = const T __attribute__((address_space(4)))*;
+template <typename T>
+__device__ inline ConstPtr<T> as_constant(const T* p)
+{
+	return (ConstPtr<T>)(unsigned long long)p;
+}
+
 constexpr __host__ __device__ int ipow(int b, int e) { return e == 0 ? 1 : b * ipow(b, e - 1); }
 
 // ------------------------------------------------------------------------------------------ fluxes

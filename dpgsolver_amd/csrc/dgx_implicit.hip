@@ -590,8 +590,7 @@ struct PrecondBlockJacobi : Precond {
 			DGX_HIP_CHECK(hipMalloc(&blocks, sizeof(double) * (size_t)c.E * nb * nb));
 			DGX_HIP_CHECK(hipMalloc(&piv, sizeof(int) * (size_t)c.E * nb));
 		}
-		for (int col = 0; col < nb; ++col) DGX_HIP_CHECK(launch_diag_col(c, u, blocks, col));
-		DGX_HIP_CHECK(launch_sub_mass(c, blocks, inv_dt, 0.0));
+		DGX_HIP_CHECK(launch_diag_blocks(c, u, inv_dt, blocks));
 		if (cap_blocks && cap_feat && cap_sigma && cap_count + c.E <= cap_capacity) {
 			const int nf = (nb + c.Np + 1 + 15) / 16 * 16;
 			DGX_HIP_CHECK(hipMemcpyAsync(cap_blocks + (size_t)cap_count * nb * nb, blocks,
@@ -642,7 +641,7 @@ struct PrecondBlockSGS : Precond {
 		if (full(c))
 			for (int col = 0; col < nb; ++col) DGX_HIP_CHECK(launch_ns_offd_col(c, u, offT, col, true));
 		else
-			for (int col = 0; col < nfv; ++col) DGX_HIP_CHECK(launch_offd_col(c, u, offT, col));
+			DGX_HIP_CHECK(launch_offd_blocks(c, u, offT));
 		if (!fp32) return hipSuccess;
 		const size_t ni = (size_t)c.E * nb * nb, no = (size_t)c.E * nf * fb * fb;
 		if (!inv32) DGX_HIP_CHECK(hipMalloc(&inv32, sizeof(float) * ni));

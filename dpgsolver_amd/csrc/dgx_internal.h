@@ -24,6 +24,7 @@ struct Ops1D {
 	T I[kMaxN * kMaxN];      // GLL -> GL interpolation
 	T IT[kMaxN * kMaxN];     // transpose of I (test-function side)
 	T DhT[kMaxN * kMaxN];    // transpose of the GL-collocated derivative
+	T DI[kMaxN * kMaxN];     // derivative of the GLL basis at the GL points
 	T Iinv[kMaxN * kMaxN];   // inverse of I (GL -> GLL)
 	T Dg[kMaxN * kMaxN];     // GLL-collocated derivative (metric nodes)
 	T B[kMaxN * kMaxN];      // Bernstein basis at the GLL nodes (Bezier -> nodal)
@@ -350,6 +351,10 @@ hipError_t launch_diag_col(Ctx& c, const double* u, double* blocks, int col);
 // column col < nv * N^(d-1) of the compact face blocks: blocks[((e * 2d + lf) * nfv + col) * nfv + row], nfv =
 // nv * N^(d-1), rows and columns on the face nodes (see MODE_OFFD)
 hipError_t launch_offd_col(Ctx& c, const double* u, double* blocks, int col);
+// every diagonal block dR_e/du_e - scale[e] M_e (scale NULL: no mass term), and every compact face block in the layout
+// of launch_offd_col (k_blocks.hip)
+hipError_t launch_diag_blocks(Ctx& c, const double* u, const double* scale, double* blocks);
+hipError_t launch_offd_blocks(Ctx& c, const double* u, double* offT);
 hipError_t launch_expand_face_blocks(Ctx& c, const double* cT, double* full);   // compact -> full nb x nb (2-D)
 // block-sparse assembly: values[slot[e]] (+)= src[e * stride + off] (slot < 0: skipped)
 hipError_t launch_bsr_place(hipStream_t s, const double* src, size_t stride, size_t off, const int* slot, double* vals,

@@ -149,6 +149,7 @@ void build_ops(int d, int p, Ops1D<double>& o, Ops1D<float>& o32)
 			o.DhT[r * N + c] = Dh[c * N + r];
 			o.Iinv[r * N + c] = Iinv[r * N + c];
 			o.Dg[r * N + c] = Dg[r * N + c];
+			o.DI[r * N + c] = D1[r * N + c];
 		}
 	// Bernstein at GLL nodes
 	for (int r = 0; r < N; ++r) {
@@ -187,7 +188,7 @@ void build_ops(int d, int p, Ops1D<double>& o, Ops1D<float>& o32)
 	// FP32 copy
 	auto cp = [](const double* s, float* t, int n) { for (int i = 0; i < n; ++i) t[i] = (float)s[i]; };
 	const int M2 = kMaxN * kMaxN;
-	cp(o.I, o32.I, M2); cp(o.IT, o32.IT, M2); cp(o.DhT, o32.DhT, M2); cp(o.Iinv, o32.Iinv, M2);
+	cp(o.I, o32.I, M2); cp(o.IT, o32.IT, M2); cp(o.DI, o32.DI, M2); cp(o.DhT, o32.DhT, M2); cp(o.Iinv, o32.Iinv, M2);
 	cp(o.Dg, o32.Dg, M2); cp(o.B, o32.B, M2); cp(o.Binv, o32.Binv, M2);
 	cp(o.Ext[0], o32.Ext[0], 2 * kMaxN); cp(o.Lift[0], o32.Lift[0], 2 * kMaxN);
 	cp(o.w, o32.w, kMaxN); cp(o.wgll, o32.wgll, kMaxN);

@@ -19,7 +19,8 @@ static hipError_t dispatch_dual(Ctx& c, const RhsArgs<S, R>& a)
 		if (flux == DGX_FLUX_LF) return run_rhs<S, R, 2, NN, DGX_PDE_EULER, DGX_FLUX_LF, MODE>(a, c.stream);            \
 		return run_rhs<S, R, 2, NN, DGX_PDE_EULER, DGX_FLUX_ROE, MODE>(a, c.stream);                                    \
 	}
-	DGX_DCASE(2) DGX_DCASE(3) DGX_DCASE(4) DGX_DCASE(5)
+	// QUAD blocks: k_blocks.hip
+	if constexpr (MODE == MODE_JVP) { DGX_DCASE(2) DGX_DCASE(3) DGX_DCASE(4) DGX_DCASE(5) }
 #undef DGX_DCASE
 	// 3-D (HEX): J v, the diagonal blocks and the face blocks, FP64 dual numbers
 #define DGX_DCASE3(NN)                                                                                   \
