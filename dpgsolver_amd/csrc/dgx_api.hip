@@ -1165,7 +1165,9 @@ dgx_status dgx_ssp_rk3_step(dgx_ctx* h, double* u, double dt, int positivity, do
 	const bool pos = positivity && c.cfg.pde != DGX_PDE_ADVECTION;
 	if (pos && c.hp && !c.hp->tri.empty()) return DGX_ERR_UNSUPPORTED;   // the limiter is built for QUAD/HEX only
 	if (pos) DGX_TRY(dgx::launch_fill_i32(c.stream, c.dstatus, 1, 0));
-	for (int rk = 0; rk < 3; ++rk) {
+	const bool fused = !c.hp && dgx::rk_fused(c);
+	if (fused) DGX_TRY(dgx::launch_rk3_fused(c, u, c.u0, c.rtmp, dt, pos, c.dstatus, c.dmax));
+	for (int rk = 0; rk < 3 && !fused; ++rk) {
 		DGX_TRY(dgx::launch_fill_u64(c.stream, c.dmax, 1, 0ull));
 		if (c.hp) {
 			// every group's residual from the stage's state, then every group's stage update
@@ -1302,6 +1304,7 @@ dgx_status dgx_graph_create_rk3(dgx_ctx* h, double* u, double dt, int positivity
 	g->rk3 = true;
 	g->positivity = positivity && c.cfg.pde != DGX_PDE_ADVECTION;
 	const dgx_status st = capture_graph(h, g, [&]() -> hipError_t {
+		if (dgx::rk_fused(c)) return dgx::launch_rk3_fused(c, u, c.u0, c.rtmp, dt, g->positivity, c.dstatus, c.dmax);
 		for (int rk = 0; rk < 3; ++rk) {
 			DGX_HIP_CHECK(dgx::launch_fill_u64(c.stream, c.dmax, 1, 0ull));
 			DGX_HIP_CHECK(dgx::launch_rhs64(c, u, c.rtmp, dgx::MODE_RHS_MINV, c.dmax));

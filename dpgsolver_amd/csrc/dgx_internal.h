@@ -322,6 +322,11 @@ hipError_t launch_positivity(Ctx& c, double* u, int* status);
 hipError_t launch_maxabs(Ctx& c, const double* r, size_t n, unsigned long long* dmax);
 hipError_t launch_convert(const double* src, float* dst, size_t n, hipStream_t s);
 hipError_t launch_convert_back(const float* src, double* dst, size_t n, hipStream_t s);
+// one SSP-RK3 step in three launches, out of place through ua and ub (E*Np*nv each); *dmax receives max |M^-1 R| of the
+// last stage; rk_fused: whether this context's step can take them
+bool rk_fused(const Ctx& c);
+hipError_t launch_rk3_fused(Ctx& c, double* u, double* ua, double* ub, double dt, bool positivity, int* status,
+                            unsigned long long* dmax);
 hipError_t launch_rk_stage(Ctx& c, double* u, const double* r, double dt, int stage);
 // the same with the stage-0 copy in u0 (E*Np*nv doubles) instead of c.u0
 hipError_t launch_rk_stage_buf(Ctx& c, double* u, double* u0, const double* r, double dt, int stage);

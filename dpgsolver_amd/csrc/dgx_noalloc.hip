@@ -62,7 +62,9 @@ extern "C" dgx_status dgx_ssp_rk3_step_noalloc(dgx_ctx* h, double* u, double dt,
 	const bool pos = positivity && c.cfg.pde != DGX_PDE_ADVECTION;
 	// the array keeps the previous call's contents: clear the flag and the max-norm slot with fill kernels
 	if (pos && dgx::launch_fill_i32(c.stream, flag, 1, 0) != hipSuccess) return DGX_ERR_HIP;
-	for (int rk = 0; rk < 3; ++rk) {
+	const bool fused = dgx::rk_fused(c);
+	if (fused && dgx::launch_rk3_fused(c, u, u0, r, dt, pos, flag, dmax) != hipSuccess) return DGX_ERR_HIP;
+	for (int rk = 0; rk < 3 && !fused; ++rk) {
 		if (dgx::launch_fill_u64(c.stream, dmax, 1, 0ull) != hipSuccess ||
 		    dgx::launch_rhs64(c, u, r, dgx::MODE_RHS_MINV, dmax) != hipSuccess ||
 		    dgx::launch_rk_stage_buf(c, u, u0, r, dt, rk) != hipSuccess)

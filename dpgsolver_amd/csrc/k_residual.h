@@ -47,7 +47,12 @@ __device__ inline Dual32 operator*(float a, Dual32 b) { return Dual32(a * b.v, a
 // transposed: out[((e * 2d + lf) * NFV + col) * NFV + rho].
 // MODE_VOL / MODE_FACE: the volume term alone (compute_volume_rlhs_dg) or the face term alone
 // (compute_face_rlhs_dg), added into out (the reference accumulates both into a pre-zeroed rhs).
-enum { MODE_JVP = 5, MODE_DIAG = 6, MODE_PERT = 7, MODE_OFFD = 8, MODE_VOL = 9, MODE_FACE = 10 };
+// MODE_RK / MODE_RK_POS: one SSP-RK3 stage, out = the stage's combination of base, u and dt M^-1 R(u)
+// (time_step_ssp_rk_33, solve_explicit.c:276-295), MODE_RK_POS then with the positivity limiter
+// (enforce_positivity_highorder, solve.c:187-233) on the element while it is in LDS.  out must not be u: other
+// elements read their traces from u.  base may be out.
+enum { MODE_JVP = 5, MODE_DIAG = 6, MODE_PERT = 7, MODE_OFFD = 8, MODE_VOL = 9, MODE_FACE = 10, MODE_RK = 11,
+       MODE_RK_POS = 12 };
 
 template <typename S, typename R>
 struct RhsArgs {
@@ -68,7 +73,12 @@ struct RhsArgs {
 	int col;              // MODE_DIAG column (local dof)
 	int grid;             // workgroups of the launch: 0 = one per element block, else a persistent grid
 	unsigned long long* dmax;
+	unsigned long long* clear;  // MODE_RK*: max-norm slot that this stage sets to zero (or NULL)
 	const double* mass_scale;   // MODE_JVP: out = J v - mass_scale[e] M_e v when not NULL
+	const Real* base;     // MODE_RK*: the step's initial state
+	double dt;
+	int stage;            // 0, 1, 2
+	int* status;          // MODE_RK_POS: |= 1 when an element's mean density or pressure is below EPS_PHYS
 	const Real* zf;       // 2-D variable order: lifted fluxes of the faces to elements of another order
 };
 
@@ -309,6 +319,21 @@ constexpr int rhs_epb()
 	return e > 0 ? e : 1;
 }
 
+// the maximum of the active lanes' m >= 0 (the first lanes of their wavefront) into the workgroup's slot: one LDS atomic per wavefront (of 64-bit patterns,
+// which order like non-negative values) instead of one per lane on the same word
+__device__ inline void rhs_block_max(double m, unsigned long long* slot)
+{
+	const unsigned long long act = __ballot(1);
+	unsigned long long b = (unsigned long long)__double_as_longlong(m);
+#pragma unroll
+	for (int off = 32; off > 0; off >>= 1) {
+		const int src = (int)(threadIdx.x & 63) ^ off;
+		const unsigned long long o = __shfl(b, src);
+		if ((act >> src) & 1ull) b = o > b ? o : b;
+	}
+	if ((int)(threadIdx.x & 63) == __builtin_ctzll(act)) atomicMax(slot, b);
+}
+
 template <typename S, typename R, int D, int N, int PDE, int FLUX, int MODE>
 __global__ void __launch_bounds__(256) k_rhs(RhsArgs<S, R> a)
 {
@@ -360,7 +385,7 @@ hipError_t dispatch_rhs(int d, int p, int pde, int flux, const RhsArgs<S, R>& a,
 		return run_rhs<S, R, DD, NN, DGX_PDE_ADVECTION, DGX_FLUX_UPWIND, MODE, PERSIST>(a, st);
 	DGX_CASE_EULER(2, 2) DGX_CASE_EULER(2, 3) DGX_CASE_EULER(2, 4) DGX_CASE_EULER(2, 5) DGX_CASE_EULER(2, 6)
 	DGX_CASE_EULER(3, 2) DGX_CASE_EULER(3, 3) DGX_CASE_EULER(3, 4) DGX_CASE_EULER(3, 5)
-	if constexpr (MODE != MODE_PERT) {
+	if constexpr (MODE != MODE_PERT && MODE != MODE_RK_POS) {
 		DGX_CASE_ADV(2, 2) DGX_CASE_ADV(2, 3) DGX_CASE_ADV(2, 4) DGX_CASE_ADV(2, 5) DGX_CASE_ADV(2, 6)
 	}
 #undef DGX_CASE_EULER
