@@ -267,6 +267,16 @@ struct Precond {
 	virtual ~Precond() {}
 	virtual hipError_t setup(Ctx& c, const double* u, const double* inv_dt) = 0;
 	virtual hipError_t apply(Ctx& c, const double* v, double* z) = 0;
+	// A preconditioner whose product A M^-1 maps vectors supported on part of the elements to such vectors: the Krylov
+	// space can then be built on that part alone (compact vectors of reduced_size values).
+	//   reduced_start:    z with r - A z supported there, v2 = that residual;
+	//   reduced_apply:    w2 = A M^-1 v2 (z: work, E*Np*nv);
+	//   reduced_solution: z = M^-1 v2.
+	virtual bool reducible(const Ctx&) const { return false; }
+	virtual size_t reduced_size(const Ctx&) const { return 0; }
+	virtual hipError_t reduced_start(Ctx&, const double*, double*, double*) { return hipErrorInvalidValue; }
+	virtual hipError_t reduced_apply(Ctx&, const double*, double*, double*) { return hipErrorInvalidValue; }
+	virtual hipError_t reduced_solution(Ctx&, const double*, double*) { return hipErrorInvalidValue; }
 };
 Precond* make_learned_precond(Ctx& c);  // nullptr when no model is attached
 
