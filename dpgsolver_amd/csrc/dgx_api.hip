@@ -417,6 +417,9 @@ hipError_t hp_barrier(dgx::HpData& H, hipStream_t main)
 	return e != hipSuccess ? e : dgx::hp_fork(H, main);
 }
 
+// whether no face joins two orders or types: then no kernel between the groups reads gradient traces
+bool ns_groups_alone(const dgx::HpData& H) { return H.tri.empty() && H.Fnc == 0; }
+
 // Variable-order and mixed-type residuals (FP64). Navier-Stokes: every group's gradient traces (TRI: and state
 // traces), the faces between orders or types (lifted gradients and fluxes; one launch per face-point count),
 // every group's residual (+ M^-1 and max-norm). Euler: the TRI state traces, the faces, every group's residual.
@@ -433,6 +436,21 @@ dgx_status hp_rhs64(Ctx& c, const double* u, double* r, int mode, unsigned long 
 	const bool minv = (mode == dgx::MODE_RHS_MINV);
 	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		const double mu = c.cfg.mu, Pr = c.cfg.Pr;
+		// no faces between orders or types: each group's whole residual, as on a mesh of its order alone
+		const bool alone = ns_groups_alone(H);
+		auto residual = [&](size_t g, Ctx& s) -> hipError_t {
+			double* rg = r + H.u_off[g];
+			hipError_t e = dgx::launch_rhs_ns_phase(s, u + H.u_off[g], rg, alone ? 0 : 2);
+			if (e != hipSuccess || mode != dgx::MODE_RHS_MINV) return e;
+			e = dgx::launch_minv(s, rg);
+			if (e == hipSuccess && dmax) e = dgx::launch_maxabs(s, rg, ndof(s), dmax);
+			return e;
+		};
+		if (alone) {
+			DGX_TRY(on_groups(c, residual));
+			DGX_TRY(dgx::hp_join(H, c.stream));
+			return DGX_OK;
+		}
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
 		for (size_t t = 0; t < H.tri.size(); ++t)
 			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 1, H.lane[H.tri_lane[t]]));
@@ -444,14 +462,7 @@ dgx_status hp_rhs64(Ctx& c, const double* u, double* r, int mode, unsigned long 
 			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 2, H.lane[H.tri_lane[t]]));
 			if (minv) DGX_TRY(dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, H.lane[H.tri_lane[t]]));
 		}
-		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) -> hipError_t {
-			double* rg = r + H.u_off[g];
-			hipError_t e = dgx::launch_rhs_ns_phase(s, u + H.u_off[g], rg, 2);
-			if (e != hipSuccess || mode != dgx::MODE_RHS_MINV) return e;
-			e = dgx::launch_minv(s, rg);
-			if (e == hipSuccess && dmax) e = dgx::launch_maxabs(s, rg, ndof(s), dmax);
-			return e;
-		}));
+		DGX_TRY(on_groups(c, residual));
 	} else {
 		if (H.tri.empty()) {
 			DGX_TRY(dgx::launch_hp_faces64(c, u));
@@ -478,6 +489,11 @@ dgx_status hp_rhs32(Ctx& c, const float* u, float* r)
 	DGX_TRY(dgx::hp_fork(H, c.stream));
 	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		const double mu = c.cfg.mu, Pr = c.cfg.Pr;
+		if (ns_groups_alone(H)) {
+			DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 0); }));
+			DGX_TRY(dgx::hp_join(H, c.stream));
+			return DGX_OK;
+		}
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
 		for (size_t t = 0; t < H.tri.size(); ++t)
 			DGX_TRY(dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 1, H.lane[H.tri_lane[t]]));
@@ -512,7 +528,9 @@ dgx_status hp_rhs_mixed(Ctx& c, const double* u, float* r)
 	dgx::HpData& H = *c.hp;
 	if (!H.tri.empty()) return DGX_ERR_UNSUPPORTED;   // TRI elements: FP64 only
 	DGX_TRY(dgx::hp_fork(H, c.stream));
-	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
+	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES && ns_groups_alone(H)) {
+		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 0); }));
+	} else if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
 		DGX_TRY(hp_barrier(H, c.stream));
 		DGX_TRY(dgx::launch_hp_faces_mixed(c, u));

@@ -13,6 +13,8 @@
 // xi = -1 / +1 is Lift_side = I^-T e_side, so the face part of that trace is q(a) kappa(a) with the geometric
 // factor kappa(a) = sum_c Lift_side(c)^2 / (w_c J(c, a)).
 //
+// The residual of a mesh without faces between orders or types: k_ns_own and k_ns_add.  The linearisation, and the groups
+// of a mesh that has such faces:
 //   k_ns_gv:  per element, the face traces of G_v and kappa (its own state and geometry only).
 //   k_rhs_ns: G_v again, the face products q from the own and neighbour traces, G for the volume flux
 //     F_euler(s) + fv(s, G) (fv the negated viscous flux, compute_Flux_navier_stokes_0,
@@ -228,6 +230,325 @@ __global__ void __launch_bounds__(128) k_ns_gv(NsArgs<S> a)
 			a.kap[(size_t)e * 4 * N + item] = acc;
 		}
 	}
+}
+
+// The residual without faces between orders (k_rhs_ns with the gradient kernel before it stays for the linearisation and
+// for meshes with such faces, whose kernels read the gradient traces).
+//
+// The central viscous flux of a face is the mean of two one-sided fluxes, and a side's needs only that side's gradient:
+// its own volume gradient and the face product q of the two state traces.  So each element computes everything but its
+// neighbours' halves, and writes its own half (three values per face point, J_f n . fv / 2 in the neighbour's sign) for
+// them; k_ns_add then lifts the neighbours' halves onto the face nodes.  A boundary face has no other half.
+// Bound by memory: per element of QUAD p = 3 FP64 state, geometry, residual and halves are 2.2 KB here and 1.1 KB in
+// k_ns_add, where the gradient traces (1 KB written, 2 KB read back) made it 6.5 KB; the volume gradient is computed
+// once instead of twice.  448 x 448, Roe, FP64: 306 -> 242 us (222 here: the FP64 pipe takes 138, LDS 122 of them).
+// LDS regions change hands: the face traces (own and neighbour) become the face products in place, the volume gradient
+// becomes the weighted fluxes, the GLL state becomes the face fluxes.
+template <typename S, int N, int FLUX, bool PERT, bool SUTH>
+__global__ void __launch_bounds__(128) k_ns_own(NsArgs<S> a, S* __restrict__ half)
+{
+	using G = typename NsArgs<S>::G;
+	constexpr int Np = N * N, EPB = ns_epb<S, N>(), TS = 4 * kNsNV * N;
+	constexpr int GS = 2 * kNsNV * Np;
+	const S eta = S(1.01 * 4.0);
+	__shared__ NsBlock<S, N> B;
+	__shared__ S T[EPB][2 * TS];   // traces at the face GL points, own ordering: own [lf][v][a], neighbour; then q_0, q_1
+	__shared__ S GX[EPB][GS];      // G_v at the GL nodes [d][v][node]; then W fr_d
+	__shared__ S WJi[EPB][Np];     // 1 / (w_c0 w_c1 J)
+	constexpr int UR = NsBlock<S, N>::UR;
+	S(*RES)[UR] = B.U;             // J_f times the face flux without the neighbour's viscous half, own ordering and sign
+	const int sl = threadIdx.x / Np, t = threadIdx.x % Np;
+	const int e = blockIdx.x * EPB + sl;
+	const bool valid = sl < EPB && e < a.E;
+	const int slc = sl < EPB ? sl : 0;
+	ns_load<S, N, PERT, kNsRhs>(B, a, slc, t, valid ? e : 0, valid);
+	const int c0 = t % N, c1 = t / N;
+	// the neighbours' face nodes, one value per lane, into the neighbour half of T in the own ordering (GLL and GL points
+	// reverse alike)
+	if (valid)
+		for (int item = t; item < 4 * N; item += Np) {
+			const int lf = item / N, o = item % N;
+			const ElemFace f = B.ef[slc][lf];
+			if (f.en < 0) continue;
+			const int b = B.perm[(f.packed >> 8) & 7][o];
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) {
+				const size_t gn = ((size_t)f.en * kNsNV + v) * Np + ns_face_node<N>(f.packed & 15, b);
+				if constexpr (PERT) T[slc][TS + (lf * kNsNV + v) * N + o] = S(a.u64[gn] - B.C[slc][v]);
+				else T[slc][TS + (lf * kNsNV + v) * N + o] = a.u[gn];
+			}
+		}
+	S g[2 * kNsNV];
+	if (valid) {
+		ns_volume_gradient<S, N>(B, a, slc, t, e, g);
+#pragma unroll
+		for (int k = 0; k < 2 * kNsNV; ++k) GX[slc][k * Np + t] = g[k];
+		WJi[slc][t] = trcp(B.w[c0] * B.w[c1] * a.detJ[(size_t)e * Np + t]);
+	}
+	__syncthreads();
+	constexpr int IT = (4 * N + Np - 1) / Np;
+	S own[IT][kNsNV], nb[IT][kNsNV];
+#pragma unroll
+	for (int k = 0; k < IT; ++k) {
+		const int item = t + k * Np;
+		if (!valid || item >= 4 * N) continue;
+		const int lf = item / N, o = item % N;
+#pragma unroll
+		for (int v = 0; v < kNsNV; ++v) {
+			S ao = S(0.0), an = S(0.0);
+#pragma unroll
+			for (int b = 0; b < N; ++b) {
+				ao += B.I[o * N + b] * B.U[slc][v * Np + ns_face_node<N>(lf, b)];
+				an += B.I[o * N + b] * T[slc][TS + (lf * kNsNV + v) * N + b];
+			}
+			own[k][v] = ao;
+			nb[k][v] = an;
+		}
+	}
+	__syncthreads();   // the GLL state and the neighbour nodes are dead: RES and the face products take their places
+#pragma unroll
+	for (int k = 0; k < IT; ++k) {
+		const int item = t + k * Np;
+		if (!valid || item >= 4 * N) continue;
+		const int lf = item / N, o = item % N, fd = lf >> 1, es = lf & 1;
+		const ElemFace fc = B.ef[slc][lf];
+		const int side = (fc.packed >> 4) & 1, bc = (fc.packed >> 12) & 15;
+		const int il = side == 0 ? o : B.perm[(fc.packed >> 8) & 7][o];   // left ordering
+		const bool wall = fc.en < 0;
+		const bool nf_provided = bc == DGX_BC_NOSLIP_ADIABATIC || bc == DGX_BC_NOSLIP_DIABATIC;
+		const G* nJ = a.nJ + ((size_t)fc.f * N + il) * 2;
+		const G nJ0 = nJ[0], nJ1 = nJ[1];
+		if (wall) {
+			// boundary state from the own trace (PERT: in FP64 from c_e + delta, back to a delta)
+			const double Jd = tsqrt((double)nJ0 * nJ0 + (double)nJ1 * nJ1);
+			double xy[2] = { 0.0, 0.0 };
+			if (bc == DGX_BC_NOSLIP_ROTATING) {
+				xy[0] = a.wall_xy[((size_t)fc.f * N + il) * 2];
+				xy[1] = a.wall_xy[((size_t)fc.f * N + il) * 2 + 1];
+			}
+			if constexpr (PERT) {
+				double so[kNsNV], sb[kNsNV];
+				const double nd[2] = { (double)nJ0 / Jd, (double)nJ1 / Jd };
+#pragma unroll
+				for (int v = 0; v < kNsNV; ++v) so[v] = B.C[slc][v] + (double)own[k][v];
+				ns_wall_state<double>(bc, so, nd, a.bc_prim, a.walls, xy, sb);
+#pragma unroll
+				for (int v = 0; v < kNsNV; ++v) nb[k][v] = S(sb[v] - B.C[slc][v]);
+			} else {
+				S sb[kNsNV];
+				const S n2[2] = { S((double)nJ0 / Jd), S((double)nJ1 / Jd) };
+				ns_wall_state<S>(bc, own[k], n2, a.bc_prim, a.walls, xy, sb);
+#pragma unroll
+				for (int v = 0; v < kNsNV; ++v) nb[k][v] = sb[v];
+			}
+		}
+		// the own side's gradient: trace(G_v) + eta kappa q, q = J_f n (s_R - s_L) / 2
+		S kap = S(0.0), gf[2 * kNsNV] = {};
+#pragma unroll
+		for (int c = 0; c < N; ++c) {
+			const int node = fd == 0 ? c + N * o : o + N * c;
+			const S lc = B.Lift[es][c];
+			kap += lc * lc * WJi[slc][node];
+#pragma unroll
+			for (int q = 0; q < 2 * kNsNV; ++q) gf[q] += lc * GX[slc][q * Np + node];
+		}
+		kap = kap * B.w[o];   // sum_c Lift(c)^2 / (w_c J) = w_a sum_c Lift(c)^2 WJi
+		S sL[kNsNV], sR[kNsNV];
+#pragma unroll
+		for (int v = 0; v < kNsNV; ++v) {
+			sL[v] = side == 0 ? own[k][v] : nb[k][v];
+			sR[v] = side == 0 ? nb[k][v] : own[k][v];
+			const S dl = S(0.5) * (sR[v] - sL[v]);
+			const S q0 = nJ0 * dl, q1 = nJ1 * dl;
+			T[slc][(lf * kNsNV + v) * N + o] = q0;
+			T[slc][TS + (lf * kNsNV + v) * N + o] = q1;
+			gf[v] += eta * kap * q0;
+			gf[kNsNV + v] += eta * kap * q1;
+		}
+		const S sgn = side == 0 ? S(1.0) : S(-1.0);
+		S hv[kNsNV];   // J_f n . fv / 2 of the own side
+		if constexpr (PERT) {
+			// FP64 states c_e + delta and fluxes; the normal Euler flux of c_e is subtracted before rounding
+			const double* ce = B.C[slc];
+			double cL[kNsNV], cR[kNsNV], so[kNsNV], gd[2 * kNsNV], fdn[kNsNV], cn[kNsNV], fv[2 * kNsNV], cu[2];
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) {
+				cL[v] = ce[v] + (double)sL[v];
+				cR[v] = ce[v] + (double)sR[v];
+				so[v] = side == 0 ? cL[v] : cR[v];
+			}
+#pragma unroll
+			for (int q = 0; q < 2 * kNsNV; ++q) gd[q] = (double)gf[q];
+			const double Jd = tsqrt((double)nJ0 * nJ0 + (double)nJ1 * nJ1), Ji = trcp(Jd);
+			const double nd[2] = { (double)nJ0 * Ji, (double)nJ1 * Ji };
+			if constexpr (FLUX == DGX_FLUX_LF) numflux_lf<double, 2>(cL, cR, nd, fdn);
+			else numflux_roe<double, 2>(cL, cR, nd, fdn);
+			const double ci = 1.0 / ce[0];
+			cu[0] = ce[1] * ci;
+			cu[1] = ce[2] * ci;
+			const double pc = kGM1 * (ce[3] - 0.5 * ce[0] * (cu[0] * cu[0] + cu[1] * cu[1]));
+			euler_normal_flux<double, 2>(ce, cu, pc, nd, cn);
+			ns_viscous_flux2<double>(so, gd, ns_mu<SUTH, double>(so, (double)a.mu, a.r_s), (double)a.Pr, fv);
+			double fw[2 * kNsNV];
+			if (wall) ns_viscous_flux2<double>(cR, gd, ns_mu<SUTH, double>(cR, (double)a.mu, a.r_s), (double)a.Pr, fw);
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) {
+				double vis = 0.5 * (nd[0] * fv[0 + 2 * v] + nd[1] * fv[1 + 2 * v]);
+				hv[v] = S(vis * Jd);
+				if (wall) vis += 0.5 * (nd[0] * fw[0 + 2 * v] + nd[1] * fw[1 + 2 * v]);
+				// no-slip flux walls: the energy flux is the provided one (numerical_flux_central_T.c:222-230)
+				const double tot = (nf_provided && v == kNsNV - 1) ? a.walls.nfE : fdn[v] + vis;
+				RES[slc][(lf * kNsNV + v) * N + o] = sgn * S((tot - cn[v]) * Jd);
+			}
+		} else {
+			const S Jf = tsqrt(nJ0 * nJ0 + nJ1 * nJ1), Jfi = trcp(Jf);
+			const S nu[2] = { nJ0 * Jfi, nJ1 * Jfi };
+			S nnf[kNsNV], fv[2 * kNsNV], fw[2 * kNsNV];
+			if constexpr (FLUX == DGX_FLUX_LF) numflux_lf<S, 2>(sL, sR, nu, nnf);
+			else numflux_roe<S, 2>(sL, sR, nu, nnf);
+			ns_viscous_flux2<S>(own[k], gf, ns_mu<SUTH, S>(own[k], a.mu, a.r_s), a.Pr, fv);
+			if (wall) ns_viscous_flux2<S>(nb[k], gf, ns_mu<SUTH, S>(nb[k], a.mu, a.r_s), a.Pr, fw);
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) {
+				S vis = S(0.5) * (nu[0] * fv[0 + 2 * v] + nu[1] * fv[1 + 2 * v]);
+				hv[v] = vis * Jf;
+				if (wall) vis += S(0.5) * (nu[0] * fw[0 + 2 * v] + nu[1] * fw[1 + 2 * v]);
+				const S tot = (nf_provided && v == kNsNV - 1) ? S(a.walls.nfE) : nnf[v] + vis;
+				RES[slc][(lf * kNsNV + v) * N + o] = sgn * (tot * Jf);
+			}
+		}
+		// the other side tests with the opposite sign
+#pragma unroll
+		for (int v = 1; v < kNsNV; ++v) half[(((size_t)e * 4 + lf) * 3 + v - 1) * N + o] = -sgn * hv[v];
+	}
+	__syncthreads();   // face products and fluxes are complete, the gradient traces taken
+	if (valid) {
+		// G = G_v + sum_faces G_f at this node, then the volume flux
+		S f[2 * kNsNV];
+		const S wq = B.w[c0] * B.w[c1], wji = WJi[slc][t];
+#pragma unroll
+		for (int lf = 0; lf < 4; ++lf) {
+			const int fd = lf >> 1, cn = fd == 0 ? c0 : c1, at = fd == 0 ? c1 : c0;
+			const S lw = B.Lift[lf & 1][cn] * B.w[at] * wji;
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) {
+				g[v] += lw * T[slc][(lf * kNsNV + v) * N + at];
+				g[kNsNV + v] += lw * T[slc][TS + (lf * kNsNV + v) * N + at];
+			}
+		}
+		if constexpr (PERT) {
+			// FP64 pointwise fluxes of c_e + V minus the Euler flux of c_e; the contractions stay in S
+			double sd[kNsNV], cd[kNsNV], gd[2 * kNsNV], fd[2 * kNsNV], fcd[2 * kNsNV], fvd[2 * kNsNV];
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) {
+				cd[v] = B.C[slc][v];
+				sd[v] = cd[v] + (double)B.V[slc][v * Np + t];
+			}
+#pragma unroll
+			for (int q = 0; q < 2 * kNsNV; ++q) gd[q] = (double)g[q];
+			euler_flux<double, 2>(sd, fd);
+			euler_flux<double, 2>(cd, fcd);
+			ns_viscous_flux2<double>(sd, gd, ns_mu<SUTH, double>(sd, (double)a.mu, a.r_s), (double)a.Pr, fvd);
+#pragma unroll
+			for (int q = 0; q < 2 * kNsNV; ++q) f[q] = S(fd[q] - fcd[q] + fvd[q]);
+		} else {
+			S s[kNsNV], fv[2 * kNsNV];
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) s[v] = B.V[slc][v * Np + t];
+			euler_flux<S, 2>(s, f);
+			ns_viscous_flux2<S>(s, g, ns_mu<SUTH, S>(s, a.mu, a.r_s), a.Pr, fv);
+#pragma unroll
+			for (int q = 0; q < 2 * kNsNV; ++q) f[q] += fv[q];
+		}
+		const G* m = a.met + (size_t)e * 4 * Np;
+#pragma unroll
+		for (int d0 = 0; d0 < 2; ++d0)
+#pragma unroll
+			for (int v = 0; v < kNsNV; ++v) {
+				// fr_d0 = sum_d1 m(d1, d0) f_d1, m[(i + 2 j)] = J dxi_j / dx_i
+				const S fr = m[(0 + 2 * d0) * Np + t] * f[0 + 2 * v] + m[(1 + 2 * d0) * Np + t] * f[1 + 2 * v];
+				GX[slc][(d0 * kNsNV + v) * Np + t] = wq * fr;
+			}
+	}
+	__syncthreads();
+	S z[kNsNV];
+	if (valid) {
+		// weak divergence sum_d Dh_d^T (W fr_d), minus the face lifts, at the GL nodes
+#pragma unroll
+		for (int v = 0; v < kNsNV; ++v) {
+			S acc = S(0.0);
+#pragma unroll
+			for (int mm = 0; mm < N; ++mm) {
+				acc += B.DhT[c0 * N + mm] * GX[slc][v * Np + mm + N * c1];
+				acc += B.DhT[c1 * N + mm] * GX[slc][(kNsNV + v) * Np + c0 + N * mm];
+			}
+#pragma unroll
+			for (int lf = 0; lf < 4; ++lf) {
+				const int fd = lf >> 1, cn = fd == 0 ? c0 : c1, at = fd == 0 ? c1 : c0;
+				acc -= B.Lift[lf & 1][cn] * B.w[at] * RES[slc][(lf * kNsNV + v) * N + at];
+			}
+			z[v] = acc;
+			B.V[slc][v * Np + t] = acc;   // (the GL state: every lane has read its own value)
+		}
+	}
+	__syncthreads();
+	// back to the GLL test functions: Ibar^T = I^T along s, then along r
+	if (valid)
+#pragma unroll
+		for (int v = 0; v < kNsNV; ++v) {
+			S acc = S(0.0);
+#pragma unroll
+			for (int mm = 0; mm < N; ++mm) acc += B.I[mm * N + c1] * B.V[slc][v * Np + c0 + N * mm];
+			GX[slc][v * Np + t] = acc;
+		}
+	__syncthreads();
+	if (valid)
+#pragma unroll
+		for (int v = 0; v < kNsNV; ++v) {
+			S acc = S(0.0);
+#pragma unroll
+			for (int mm = 0; mm < N; ++mm) acc += B.I[mm * N + c0] * GX[slc][v * Np + mm + N * c1];
+			a.out[((size_t)e * kNsNV + v) * Np + t] = acc;
+		}
+}
+
+// r -= the neighbours' viscous halves, lifted onto the face nodes: sum_a I[a][b] w_a half(a) at node b of the face.
+// Bound by memory, 47 us at 448 x 448, p = 3 (1.1 KB an element).  Halves to LDS first, one face point per lane: gathered
+// by every lane of a face they took 142 us of address work.
+template <typename S, int N>
+__global__ void __launch_bounds__(256) k_ns_add(const ElemFace* __restrict__ ef, const Ops1D<S>* __restrict__ ops,
+                                                const S* __restrict__ half, S* __restrict__ r, int E)
+{
+	constexpr int Np = N * N, EPB = 256 / Np;
+	__shared__ S sIw[Np], sh[EPB][4][3][N];   // I[a][b] w_a; the neighbours' halves, own ordering
+	const int sl = threadIdx.x / Np, t = threadIdx.x % Np, e = blockIdx.x * EPB + sl;
+	const bool valid = sl < EPB && e < E;
+	for (int i = threadIdx.x; i < Np; i += 256) sIw[i] = ops->I[i] * ops->w[i / N];
+	if (valid)
+		for (int item = t; item < 4 * N; item += Np) {
+			const int lf = item / N, o = item % N;
+			const ElemFace f = ef[(size_t)e * 4 + lf];
+			const int q = ((f.packed >> 8) & 7) ? N - 1 - o : o;   // 2-D: the orientation bits are 0 or 2 (reversed)
+#pragma unroll
+			for (int v = 0; v < 3; ++v)
+				sh[sl][lf][v][o] = f.en >= 0 ? half[(((size_t)f.en * 4 + (f.packed & 15)) * 3 + v) * N + q] : S(0.0);
+		}
+	__syncthreads();
+	const int c0 = t % N, c1 = t / N;
+	if (!valid || (c0 != 0 && c0 != N - 1 && c1 != 0 && c1 != N - 1)) return;
+	S acc[3] = {};
+#pragma unroll
+	for (int lf = 0; lf < 4; ++lf) {
+		const int fd = lf >> 1;
+		if ((fd == 0 ? c0 : c1) != ((lf & 1) ? N - 1 : 0)) continue;
+		const int b = fd == 0 ? c1 : c0;
+#pragma unroll
+		for (int q = 0; q < N; ++q)
+#pragma unroll
+			for (int v = 0; v < 3; ++v) acc[v] += sIw[q * N + b] * sh[sl][lf][v][q];
+	}
+#pragma unroll
+	for (int v = 0; v < 3; ++v) r[((size_t)e * kNsNV + 1 + v) * Np + t] -= acc[v];
 }
 
 template <typename S, int N, int FLUX, bool PERT, int MODE, bool SUTH>
@@ -560,8 +881,10 @@ __global__ void __launch_bounds__(128) k_rhs_ns(NsArgs<S> a)
 		}
 }
 
-// phase 0: both kernels; 1: the gradient traces only; 2: the residual only (variable-order meshes run the
-// face kernel between orders in between)
+// phase 0: the whole residual; 1: the gradient traces only; 2: the residual only (variable-order meshes run the
+// face kernel between orders in between).  The residual needs no other element's gradient traces in phase 0, so it takes
+// k_ns_own and k_ns_add there (242 us against 306 at 448 x 448, p = 3, FP64); the dual numbers of the linearisation keep
+// the gradient-trace kernels, whose traces every block column reads.
 template <typename S, int N, bool PERT, int MODE>
 hipError_t run_ns(Ctx& c, const NsArgs<S>& a, int phase)
 {
@@ -571,6 +894,26 @@ hipError_t run_ns(Ctx& c, const NsArgs<S>& a, int phase)
 	// residual launch per local face (blockIdx.y) seeded through that face's neighbour
 	constexpr int GVMODE = (MODE == kNsOffd) ? kNsDiag : MODE;
 	const dim3 rgrid(grid, MODE == kNsOffd ? 4 : 1);
+	if constexpr (MODE == kNsRhs) {
+		if (phase == 0) {   // one order, no faces between orders: the gradient-trace buffer holds the viscous halves
+			const bool lf = c.cfg.num_flux == DGX_FLUX_LF;
+			S* half = a.gvt;
+#define DGX_NS_OWN(FL, SU) hipLaunchKernelGGL((k_ns_own<S, N, FL, PERT, SU>), dim3(grid), dim3(EPB * Np), 0, c.stream, a, half)
+			if (a.sutherland) {
+				if (lf) DGX_NS_OWN(DGX_FLUX_LF, true);
+				else DGX_NS_OWN(DGX_FLUX_ROE, true);
+			} else {
+				if (lf) DGX_NS_OWN(DGX_FLUX_LF, false);
+				else DGX_NS_OWN(DGX_FLUX_ROE, false);
+			}
+#undef DGX_NS_OWN
+			DGX_HIP_CHECK(hipGetLastError());
+			constexpr int AEPB = 256 / Np;
+			hipLaunchKernelGGL((k_ns_add<S, N>), dim3((c.E + AEPB - 1) / AEPB), dim3(256), 0, c.stream, c.elem_faces, a.ops, half,
+			                   a.out, c.E);
+			return hipGetLastError();
+		}
+	}
 	if (phase != 2) {
 		hipLaunchKernelGGL((k_ns_gv<S, N, PERT, GVMODE>), dim3(grid), dim3(EPB * Np), 0, c.stream, a);
 		DGX_HIP_CHECK(hipGetLastError());
