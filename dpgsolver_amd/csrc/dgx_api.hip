@@ -59,11 +59,6 @@ void free_hp(Ctx& c)
 	}
 	release(H->tri_ops64); release(H->tri_ops32); release(H->mfaces); release(H->mnJ); release(H->mnJ32);
 	release(H->mxy);
-	for (int k = 0; k < dgx::HpData::kLanes; ++k) {
-		if (H->lane[k]) (void)hipStreamDestroy(H->lane[k]);
-		if (H->join_ev[k]) (void)hipEventDestroy(H->join_ev[k]);
-	}
-	if (H->fork_ev) (void)hipEventDestroy(H->fork_ev);
 	delete H;
 	c.hp = nullptr;
 }
@@ -392,9 +387,9 @@ void outward_nj(const double* xyz, int N, int lf, const double* s, int ns, doubl
 	}
 }
 
-// Enqueues launch(g, s) for every order group on the group's side stream.  Each group context gets its own
-// stream back afterwards (not the caller's current one: during a graph capture that is the private capture
-// stream, destroyed when the capture ends, and a group context must never keep it).
+// Enqueues launch(g, s) for every order group on the caller's stream.  Each group context gets its own stream back
+// afterwards (during a graph capture the caller's is the private capture stream, destroyed when the capture ends, and a
+// group context must never keep it).
 template <typename F>
 hipError_t on_groups(Ctx& c, F launch)
 {
@@ -402,19 +397,12 @@ hipError_t on_groups(Ctx& c, F launch)
 	for (size_t g = 0; g < H.groups.size(); ++g) {
 		Ctx& s = H.groups[g]->c;
 		const hipStream_t own = s.stream;
-		s.stream = H.lane[H.group_lane[g]];
+		s.stream = c.stream;
 		const hipError_t e = launch(g, s);
 		s.stream = own;
 		if (e != hipSuccess) return e;
 	}
 	return hipSuccess;
-}
-
-// Every side stream waits for everything enqueued so far on the side streams.
-hipError_t hp_barrier(dgx::HpData& H, hipStream_t main)
-{
-	const hipError_t e = dgx::hp_join(H, main);
-	return e != hipSuccess ? e : dgx::hp_fork(H, main);
 }
 
 // whether no face joins two orders or types: then no kernel between the groups reads gradient traces
@@ -423,16 +411,14 @@ bool ns_groups_alone(const dgx::HpData& H) { return H.tri.empty() && H.Fnc == 0;
 // Variable-order and mixed-type residuals (FP64). Navier-Stokes: every group's gradient traces (TRI: and state
 // traces), the faces between orders or types (lifted gradients and fluxes; one launch per face-point count),
 // every group's residual (+ M^-1 and max-norm). Euler: the TRI state traces, the faces, every group's residual.
-// The launches of one phase write disjoint outputs and run concurrently on the side streams; the phases are
-// ordered by barriers.
+// All on one stream: spread over side streams, the independent launches of a phase ran side by side, but each phase
+// paid a fork and a join over the streams, 41 us, and the kernels of all but the smallest groups fill the chip alone.
+// TRI / QUAD mesh with orders 1..5, FP64, four side streams against one, us: Euler 8 x 8 274 / 97, 300 x 200 293 / 179,
+// 500 x 300 378 / 331; Navier-Stokes 287 / 182, 447 / 436, 852 / 857 (before the faces of one phase became one launch).
 dgx_status hp_rhs64(Ctx& c, const double* u, double* r, int mode, unsigned long long* dmax)
 {
 	dgx::HpData& H = *c.hp;
-	DGX_TRY(dgx::hp_fork(H, c.stream));
-	if (!H.tri.empty() && mode != dgx::MODE_RHS && mode != dgx::MODE_RHS_MINV) {
-		(void)dgx::hp_join(H, c.stream);
-		return DGX_ERR_UNSUPPORTED;
-	}
+	if (!H.tri.empty() && mode != dgx::MODE_RHS && mode != dgx::MODE_RHS_MINV) return DGX_ERR_UNSUPPORTED;
 	const bool minv = (mode == dgx::MODE_RHS_MINV);
 	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		const double mu = c.cfg.mu, Pr = c.cfg.Pr;
@@ -448,19 +434,16 @@ dgx_status hp_rhs64(Ctx& c, const double* u, double* r, int mode, unsigned long 
 		};
 		if (alone) {
 			DGX_TRY(on_groups(c, residual));
-			DGX_TRY(dgx::hp_join(H, c.stream));
 			return DGX_OK;
 		}
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
 		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 1, H.lane[H.tri_lane[t]]));
-		DGX_TRY(hp_barrier(H, c.stream));
+			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 1, c.stream));
 		if (H.tri.empty()) DGX_TRY(dgx::launch_hp_faces64(c, u));
-		else DGX_TRY(dgx::launch_mix_faces_ns64(H, c, u, H.lane[dgx::HpData::kLanes - 1]));
-		DGX_TRY(hp_barrier(H, c.stream));
+		else DGX_TRY(dgx::launch_mix_faces64(H, c, u, true));
 		for (size_t t = 0; t < H.tri.size(); ++t) {
-			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 2, H.lane[H.tri_lane[t]]));
-			if (minv) DGX_TRY(dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, H.lane[H.tri_lane[t]]));
+			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 2, c.stream));
+			if (minv) DGX_TRY(dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, c.stream));
 		}
 		DGX_TRY(on_groups(c, residual));
 	} else {
@@ -468,57 +451,47 @@ dgx_status hp_rhs64(Ctx& c, const double* u, double* r, int mode, unsigned long 
 			DGX_TRY(dgx::launch_hp_faces64(c, u));
 		} else {   // the TRI traces, then the faces
 			for (size_t t = 0; t < H.tri.size(); ++t)
-				DGX_TRY(dgx::launch_tri_trace64(H.tri[t], H.tri_ops64, u, H.lane[H.tri_lane[t]]));
-			DGX_TRY(hp_barrier(H, c.stream));
-			DGX_TRY(dgx::launch_mix_faces64(H, c, u, H.lane[dgx::HpData::kLanes - 1]));
+				DGX_TRY(dgx::launch_tri_trace64(H.tri[t], H.tri_ops64, u, c.stream));
+			DGX_TRY(dgx::launch_mix_faces64(H, c, u, false));
 		}
-		DGX_TRY(hp_barrier(H, c.stream));
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs64(s, u + H.u_off[g], r + H.u_off[g], mode, dmax); }));
 		for (size_t t = 0; t < H.tri.size(); ++t) {
-			DGX_TRY(dgx::launch_tri_rhs64(H.tri[t], H.tri_ops64, u, r, H.z64, H.lane[H.tri_lane[t]]));
-			if (minv) DGX_TRY(dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, H.lane[H.tri_lane[t]]));
+			DGX_TRY(dgx::launch_tri_rhs64(H.tri[t], H.tri_ops64, u, r, H.z64, c.stream));
+			if (minv) DGX_TRY(dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, c.stream));
 		}
 	}
-	DGX_TRY(dgx::hp_join(H, c.stream));
 	return DGX_OK;
 }
 
 dgx_status hp_rhs32(Ctx& c, const float* u, float* r)
 {
 	dgx::HpData& H = *c.hp;
-	DGX_TRY(dgx::hp_fork(H, c.stream));
 	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		const double mu = c.cfg.mu, Pr = c.cfg.Pr;
 		if (ns_groups_alone(H)) {
 			DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 0); }));
-			DGX_TRY(dgx::hp_join(H, c.stream));
 			return DGX_OK;
 		}
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
 		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 1, H.lane[H.tri_lane[t]]));
-		DGX_TRY(hp_barrier(H, c.stream));
+			DGX_TRY(dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 1, c.stream));
 		if (H.tri.empty()) DGX_TRY(dgx::launch_hp_faces32(c, u));
 		else DGX_TRY(dgx::launch_mix_faces32(H, c, u, true));
-		DGX_TRY(hp_barrier(H, c.stream));
 		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 2, H.lane[H.tri_lane[t]]));
+			DGX_TRY(dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 2, c.stream));
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 2); }));
 	} else {
 		if (H.tri.empty()) {
 			DGX_TRY(dgx::launch_hp_faces32(c, u));
 		} else {   // the TRI traces, then the faces
 			for (size_t t = 0; t < H.tri.size(); ++t)
-				DGX_TRY(dgx::launch_tri_trace32(H.tri[t], H.tri_ops32, u, H.lane[H.tri_lane[t]]));
-			DGX_TRY(hp_barrier(H, c.stream));
+				DGX_TRY(dgx::launch_tri_trace32(H.tri[t], H.tri_ops32, u, c.stream));
 			DGX_TRY(dgx::launch_mix_faces32(H, c, u, false));
 		}
-		DGX_TRY(hp_barrier(H, c.stream));
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs32(s, u + H.u_off[g], r + H.u_off[g]); }));
 		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_rhs32(H.tri[t], H.tri_ops32, u, r, H.z32, H.lane[H.tri_lane[t]]));
+			DGX_TRY(dgx::launch_tri_rhs32(H.tri[t], H.tri_ops32, u, r, H.z32, c.stream));
 	}
-	DGX_TRY(dgx::hp_join(H, c.stream));
 	return DGX_OK;
 }
 
@@ -527,21 +500,16 @@ dgx_status hp_rhs_mixed(Ctx& c, const double* u, float* r)
 {
 	dgx::HpData& H = *c.hp;
 	if (!H.tri.empty()) return DGX_ERR_UNSUPPORTED;   // TRI elements: FP64 only
-	DGX_TRY(dgx::hp_fork(H, c.stream));
 	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES && ns_groups_alone(H)) {
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 0); }));
 	} else if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
-		DGX_TRY(hp_barrier(H, c.stream));
 		DGX_TRY(dgx::launch_hp_faces_mixed(c, u));
-		DGX_TRY(hp_barrier(H, c.stream));
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 2); }));
 	} else {
 		DGX_TRY(dgx::launch_hp_faces_mixed(c, u));
-		DGX_TRY(hp_barrier(H, c.stream));
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_mixed(s, u + H.u_off[g], r + H.u_off[g]); }));
 	}
-	DGX_TRY(dgx::hp_join(H, c.stream));
 	return DGX_OK;
 }
 
@@ -1003,45 +971,6 @@ static dgx_status upload_hp_impl(dgx_ctx* h, int E, int F, const int* type, cons
 		sub->c.hp_z64 = H.z64 + H.z_off[g];
 		sub->c.hp_z32 = H.z32 + H.z_off[g];
 	}
-	// side streams, and the groups and face pairs spread over them longest first (cost ~ items x N^2)
-	for (int k = 0; k < dgx::HpData::kLanes; ++k) {
-		DGX_TRY(hipStreamCreateWithFlags(&H.lane[k], hipStreamNonBlocking));
-		DGX_TRY(hipEventCreateWithFlags(&H.join_ev[k], hipEventDisableTiming));
-	}
-	DGX_TRY(hipEventCreateWithFlags(&H.fork_ev, hipEventDisableTiming));
-	auto balance = [](const std::vector<double>& cost) {
-		std::vector<int> idx(cost.size()), lane(cost.size(), 0);
-		for (size_t i = 0; i < idx.size(); ++i) idx[i] = (int)i;
-		std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-		double load[dgx::HpData::kLanes] = {};
-		for (int i : idx) {
-			int k = 0;
-			for (int j = 1; j < dgx::HpData::kLanes; ++j)
-				if (load[j] < load[k]) k = j;
-			lane[i] = k;
-			load[k] += cost[i];
-		}
-		return lane;
-	};
-	// the QUAD and TRI groups of one phase share the streams: one balance over both (a TRI element's dense
-	// products cost about Np Nc / 3 against N^2 per QUAD element, from the measured kernel times)
-	std::vector<double> gcost(G + T), pcost(H.pairs.size());
-	for (int g = 0; g < G; ++g) gcost[g] = (double)(e_off[g + 1] - e_off[g]) * (order[g] + 1) * (order[g] + 1);
-	for (int t = 0; t < T; ++t) {
-		const int p = tri_p[t], np = (p + 1) * (p + 2) / 2, nc = p == 1 ? 3 : p == 2 ? 6 : p == 3 ? 12 : p == 4 ? 16 : 25;
-		gcost[G + t] = (double)(tri_e0[t + 1] - tri_e0[t]) * np * nc / 3.0;
-	}
-	for (size_t i = 0; i < H.pairs.size(); ++i) {
-		const int n = std::max(H.pairs[i].NL, H.pairs[i].NR);
-		pcost[i] = (double)H.pairs[i].count * n * n;
-	}
-	const std::vector<int> lanes = balance(gcost);
-	H.group_lane.assign(lanes.begin(), lanes.begin() + G);
-	H.tri_lane.assign(lanes.begin() + G, lanes.end());
-	H.pair_lane = balance(pcost);
-	std::vector<double> mcost(H.mruns.size());
-	for (size_t i = 0; i < H.mruns.size(); ++i) mcost[i] = (double)H.mruns[i].count * H.mruns[i].Nf * H.mruns[i].Nf;
-	H.mrun_lane = balance(mcost);
 	H.ready = true;
 	return DGX_OK;
 }

@@ -123,7 +123,7 @@ struct MixFace {
 	int tL, tR;          // TRI sides: the TRI group index
 };
 
-// a run of mixed faces with the same number of face points (one launch each)
+// a run of mixed faces with the same number of face points
 struct MixRun {
 	int Nf, start, count;
 };
@@ -177,13 +177,6 @@ struct HpData {
 	float* z32 = nullptr;
 	HpOps<double>* ops64 = nullptr;
 	HpOps<float>* ops32 = nullptr;
-	// Side streams (default priority) over which the independent launches of one phase are spread: the
-	// groups' kernels and the per-pair face kernels write disjoint outputs, so they run concurrently between
-	// a fork (each side stream waits for the caller's stream) and a join (the caller's stream waits for each).
-	static constexpr int kLanes = 4;
-	hipStream_t lane[kLanes] = {};
-	hipEvent_t fork_ev = nullptr;
-	hipEvent_t join_ev[kLanes] = {};
 	// TRI groups and the faces that touch a TRI element (mixed meshes)
 	std::vector<TriGroup> tri;
 	TriOps<double>* tri_ops64 = nullptr;   // device: kTriMaxP + 1 entries, indexed by p
@@ -194,15 +187,8 @@ struct HpData {
 	double* mxy = nullptr;                 // Navier-Stokes rotating walls: GL point coordinates (Fmix x kHpMaxN x 2)
 	int Fmix = 0;
 	std::vector<MixRun> mruns;             // runs of mixed faces with one Nf
-	std::vector<int> mrun_lane;            // side stream of each run (longest-first balance of count Nf^2)
-	std::vector<int> group_lane;     // side stream of each QUAD group and of each TRI group (one longest-first
-	std::vector<int> tri_lane;       // balance of the groups' costs)
-	std::vector<int> pair_lane;      // side stream of each face pair (longest-first balance of count max(NL,NR)^2)
 };
 
-// Fork / join of the variable-order side streams on `main` (the context's stream, or the capturing stream).
-hipError_t hp_fork(HpData& H, hipStream_t main);
-hipError_t hp_join(HpData& H, hipStream_t main);
 
 // Per-element face record: f, neighbour element (-1 on a boundary), and packed
 // (neighbour local face | side << 4 | ord << 8 | bc << 12).
@@ -312,14 +298,13 @@ hipError_t launch_hp_faces_mixed(Ctx& c, const double* u);   // FP64 state and f
 // mixed TRI / QUAD meshes (k_tri.hip): one TRI group's residual from its lifted face fluxes; the faces with a TRI side
 hipError_t launch_tri_rhs64(const TriGroup& g, const TriOps<double>* ops, const double* u, double* r, const double* z,
                             hipStream_t st);
-hipError_t launch_mix_faces64(const HpData& H, const Ctx& c, const double* u, hipStream_t st);
+hipError_t launch_mix_faces64(const HpData& H, const Ctx& c, const double* u, bool ns);
 // Navier-Stokes on mixed meshes: a TRI group's volume gradient and its traces (phase 1) or its residual (phase 2),
 // and the faces with a TRI side (the BR2 products y, then the lifted inviscid + viscous fluxes)
 hipError_t launch_tri_ns_phase64(const TriGroup& g, const TriOps<double>* ops, const double* u, double* r,
                                  const double* z, double mu, double Pr, int phase, hipStream_t st);
 // Euler: a TRI group's state traces at its own GL face points (before the mixed faces)
 hipError_t launch_tri_trace64(const TriGroup& g, const TriOps<double>* ops, const double* u, hipStream_t st);
-hipError_t launch_mix_faces_ns64(const HpData& H, const Ctx& c, const double* u, hipStream_t st);
 // the FP32 residual on mixed meshes (FP32 state, geometry shadows and operators; VALU kernels)
 hipError_t launch_tri_trace32(const TriGroup& g, const TriOps<float>* ops, const float* u, hipStream_t st);
 hipError_t launch_tri_rhs32(const TriGroup& g, const TriOps<float>* ops, const float* u, float* r, const float* z,

@@ -907,7 +907,6 @@ struct MixArgsT {
 	double mu, Pr;
 	NsWalls walls;                     // Navier-Stokes wall data
 	const double* wxy;                 // rotating walls: coordinates of each face's GL points (Fmix x kHpMaxN x 2)
-	int start, count;
 };
 
 // value j of variable v of one side at its own face points (TRI: trace at its GL points; QUAD: GLL face node)
@@ -992,16 +991,24 @@ __device__ inline void load_own(const MixArgsT<T>& a, int kind, int Ns, int lf, 
 	for (int v = 0; v < kNV; ++v) own[v] = side_value(a, kind, Ns, lf, uoff, el, tg, v, j);
 }
 
+// The faces of one face-point count: block `block` of the run's `count` faces from face `start` (Euler; mix_faces_ns:
+// Navier-Stokes).  The LDS of the five instances of a kernel is one buffer.
+template <typename T, int NF>
+struct MixLds {
+	MixOps<T, NF> o;
+	T F[mix_fpb(NF)][2 * kNV * NF];   // both sides' own values [side][v][i], then w J_f F [q][v]
+};
+
 template <typename T, int NF, int FLUX>
-__global__ void __launch_bounds__(256) k_mixf(MixArgsT<T> a)
+__device__ inline void mix_faces(const MixArgsT<T>& a, int start, int count, int block, void* lds)
 {
 	constexpr int LPF = mix_lpf(NF), FPB = mix_fpb(NF);
-	__shared__ MixOps<T, NF> o;
-	__shared__ T sF[FPB][2 * kNV * NF];   // both sides' own values [side][v][i], then w J_f F [q][v]
+	MixLds<T, NF>& L = *reinterpret_cast<MixLds<T, NF>*>(lds);
+	MixOps<T, NF>& o = L.o;
 	const int slot = threadIdx.x / LPF, j = threadIdx.x % LPF;
-	const int fl = blockIdx.x * FPB + slot;
-	const bool valid = fl < a.count;
-	const int fi = a.start + (valid ? fl : 0);
+	const int fl = block * FPB + slot;
+	const bool valid = fl < count;
+	const int fi = start + (valid ? fl : 0);
 	const MixFace f = a.faces[fi];
 	const bool inter = f.bc == DGX_BC_INTERIOR;
 	// every global load of this lane first (one round trip), then the operators
@@ -1014,7 +1021,7 @@ __global__ void __launch_bounds__(256) k_mixf(MixArgsT<T> a)
 		nj1 = nj[1];
 	}
 	stage_mix_ops<NF>(o, a.hops);
-	T* F = sF[slot];
+	T* F = L.F[slot];
 	if (valid && j < f.NL)
 #pragma unroll
 		for (int v = 0; v < kNV; ++v) F[v * NF + j] = oL[v];
@@ -1025,8 +1032,8 @@ __global__ void __launch_bounds__(256) k_mixf(MixArgsT<T> a)
 	const int q = j;
 	T g[kNV];
 	if (valid && j < NF) {
-		const T Jf = sqrt(nj0 * nj0 + nj1 * nj1);
-		const T nu[2] = { nj0 / Jf, nj1 / Jf };
+		const T Jf = tsqrt(nj0 * nj0 + nj1 * nj1), Jfi = trcp(Jf);
+		const T nu[2] = { nj0 * Jfi, nj1 * Jfi };
 		T sL[kNV], sR[kNV], nnf[kNV];
 		side_at_point<NF>(o, f.kL, f.NL, q, F, sL);
 		if (inter) side_at_point<NF>(o, f.kR, f.NR, f.rev ? NF - 1 - q : q, F + kNV * NF, sR);
@@ -1095,17 +1102,23 @@ __device__ inline void side_face_gradient(int kind, int Ns, int j, const T* t, c
 	for (int k = 0; k < 2 * kNV; ++k) h[k] = t[k] + eta * kr[0] * Y[k * NF + j];
 }
 
+template <typename T, int NF>
+struct MixNsLds {
+	MixOps<T, NF> o;
+	T Y[mix_fpb(NF)][2][2 * kNV * NF];   // both sides' own values [side][v][i]; then each side's y [k][i], then h
+	T Q[mix_fpb(NF)][NF * 2 * kNV];      // w q at the face points [q][k]; then w J_f F [q][v]
+};
+
 template <typename T, int NF, int FLUX>
-__global__ void __launch_bounds__(256) k_mixf_ns(MixArgsT<T> a)
+__device__ inline void mix_faces_ns(const MixArgsT<T>& a, int start, int count, int block, void* lds)
 {
 	constexpr int LPF = mix_lpf(NF), FPB = mix_fpb(NF), K8 = 2 * kNV;
-	__shared__ MixOps<T, NF> o;
-	__shared__ T sY[FPB][2][K8 * NF];   // both sides' own values [side][v][i]; then each side's y [k][i], then h
-	__shared__ T sQ[FPB][NF * K8];      // w q at the face points [q][k]; then w J_f F [q][v]
+	MixNsLds<T, NF>& L = *reinterpret_cast<MixNsLds<T, NF>*>(lds);
+	MixOps<T, NF>& o = L.o;
 	const int slot = threadIdx.x / LPF, j = threadIdx.x % LPF;
-	const int fl = blockIdx.x * FPB + slot;
-	const bool valid = fl < a.count;
-	const int fi = a.start + (valid ? fl : 0);
+	const int fl = block * FPB + slot;
+	const bool valid = fl < count;
+	const int fi = start + (valid ? fl : 0);
 	const MixFace f = a.faces[fi];
 	// the own values and normals first, then the operators
 	T oL[kNV], oR[kNV], nj0 = 1.0, nj1 = 0.0;
@@ -1120,9 +1133,9 @@ __global__ void __launch_bounds__(256) k_mixf_ns(MixArgsT<T> a)
 		nj1 = nj[1];
 	}
 	stage_mix_ops<NF>(o, a.hops);
-	T* YL = sY[slot][0];
-	T* YR = sY[slot][1];
-	T* Q = sQ[slot];
+	T* YL = L.Y[slot][0];
+	T* YR = L.Y[slot][1];
+	T* Q = L.Q[slot];
 	if (ownL)
 #pragma unroll
 		for (int v = 0; v < kNV; ++v) YL[v * NF + j] = oL[v];
@@ -1140,8 +1153,8 @@ __global__ void __launch_bounds__(256) k_mixf_ns(MixArgsT<T> a)
 		if (inter) {
 			side_at_point<NF>(o, f.kR, f.NR, qr, YL + kNV * NF, sR);
 		} else {   // the boundary state (Riemann or a no-slip wall) at this point
-			const T Jf = sqrt(nj0 * nj0 + nj1 * nj1);
-			const T nu[2] = { nj0 / Jf, nj1 / Jf };
+			const T Jfi = trcp(tsqrt(nj0 * nj0 + nj1 * nj1));
+			const T nu[2] = { nj0 * Jfi, nj1 * Jfi };
 			double xy[2] = { 0.0, 0.0 };
 			if (f.bc == DGX_BC_NOSLIP_ROTATING) {
 				xy[0] = a.wxy[((size_t)fi * kHpMaxN + q) * 2];
@@ -1196,8 +1209,8 @@ __global__ void __launch_bounds__(256) k_mixf_ns(MixArgsT<T> a)
 	wave_sync();
 	T fq[kNV];
 	if (point) {   // the flux at this face point: inviscid first, then each side's face gradient P h and viscous flux
-		const T Jf = sqrt(nj0 * nj0 + nj1 * nj1);
-		const T nu[2] = { nj0 / Jf, nj1 / Jf };
+		const T Jf = tsqrt(nj0 * nj0 + nj1 * nj1), Jfi = trcp(Jf);
+		const T nu[2] = { nj0 * Jfi, nj1 * Jfi };
 		T nnf[kNV], fvL[K8], fvR[K8];
 		if constexpr (FLUX == DGX_FLUX_LF) numflux_lf<T, 2>(sL, sR, nu, nnf);
 		else numflux_roe<T, 2>(sL, sR, nu, nnf);
@@ -1245,6 +1258,37 @@ __global__ void __launch_bounds__(256) k_mixf_ns(MixArgsT<T> a)
 	wave_sync();
 	if (ownL) lift_side<NF>(o, f.NL, j, false, false, Q, a.z + f.zL);
 	if (ownR) lift_side<NF>(o, f.NR, j, f.rev != 0, true, Q, a.z + f.zR);
+}
+
+// All runs of equal face-point count in one launch, the largest counts first: workgroups block0[i] .. of run i.  As a
+// launch each, the runs of few faces took 18 and 30 us by themselves (operators, descriptors and traces are dependent
+// loads) where they fill a few CUs.  Navier-Stokes, 500 x 300 with orders 1..5 (323 k faces), FP64: 352 -> 299 us; the
+// whole residual of an 8 x 8 mesh 182 -> 136 us.  Bound by the loads of the traces, K rows and face products (about 2.5 KB a
+// face, 160 us at the copy rate) at 12 wavefronts a CU, which 145 registers allow.
+struct MixRuns {
+	int n, Nf[kHpMaxN], start[kHpMaxN], count[kHpMaxN], block0[kHpMaxN];
+};
+
+template <typename T, int FLUX, bool NS>
+__global__ void __launch_bounds__(256) k_mix_faces(MixArgsT<T> a, MixRuns runs)
+{
+	constexpr size_t m4 = NS ? sizeof(MixNsLds<T, 4>) : sizeof(MixLds<T, 4>);
+	constexpr size_t m6 = NS ? sizeof(MixNsLds<T, 6>) : sizeof(MixLds<T, 6>);
+	constexpr size_t m2 = NS ? sizeof(MixNsLds<T, 2>) : sizeof(MixLds<T, 2>);
+	constexpr size_t m46 = m4 > m6 ? m4 : m6;
+	__shared__ alignas(16) unsigned char lds[m46 > m2 ? m46 : m2];
+	int i = 0;
+	while (i + 1 < runs.n && (int)blockIdx.x >= runs.block0[i + 1]) ++i;
+	const int start = runs.start[i], count = runs.count[i], block = blockIdx.x - runs.block0[i];
+#define DGX_MIX(NFV)                                                                    \
+	case NFV:                                                                           \
+		if constexpr (NS) mix_faces_ns<T, NFV, FLUX>(a, start, count, block, lds);      \
+		else mix_faces<T, NFV, FLUX>(a, start, count, block, lds);                      \
+		break;
+	switch (runs.Nf[i]) {
+		DGX_MIX(2) DGX_MIX(3) DGX_MIX(4) DGX_MIX(5) DGX_MIX(6)
+	}
+#undef DGX_MIX
 }
 
 // a TRI group's buffers in the precision T (FP32: the shadows of the geometry and mass data; the per-evaluation
@@ -1323,38 +1367,35 @@ MixArgsT<T> mix_args(const HpData& H, const Ctx& c, const T* u)
 	return a;
 }
 
-// the faces with a TRI side, one launch per run of equal Nf, spread over the mesh's side streams
+// the faces with a TRI side or between orders
 template <typename T>
 hipError_t launch_mix(const HpData& H, const Ctx& c, const T* u, bool ns)
 {
 	MixArgsT<T> a = mix_args<T>(H, c, u);
 	const bool lf = c.cfg.num_flux == DGX_FLUX_LF;
-	for (size_t i = 0; i < H.mruns.size(); ++i) {
-		const MixRun& run = H.mruns[i];
-		a.start = run.start;
-		a.count = run.count;
-		const hipStream_t st = H.lane[H.mrun_lane[i]];
-#define DGX_MIX(NFV)                                                                                           \
-	case NFV: {                                                                                                \
-		const dim3 grid((run.count + mix_fpb(NFV) - 1) / mix_fpb(NFV)), block(64 * kMixWaves);                 \
-		if (ns) {                                                                                              \
-			if (lf) hipLaunchKernelGGL((k_mixf_ns<T, NFV, DGX_FLUX_LF>), grid, block, 0, st, a);               \
-			else hipLaunchKernelGGL((k_mixf_ns<T, NFV, DGX_FLUX_ROE>), grid, block, 0, st, a);                 \
-		} else {                                                                                               \
-			if (lf) hipLaunchKernelGGL((k_mixf<T, NFV, DGX_FLUX_LF>), grid, block, 0, st, a);                  \
-			else hipLaunchKernelGGL((k_mixf<T, NFV, DGX_FLUX_ROE>), grid, block, 0, st, a);                    \
-		}                                                                                                      \
-		break;                                                                                                 \
-	}
-		switch (run.Nf) {
-			DGX_MIX(2) DGX_MIX(3) DGX_MIX(4) DGX_MIX(5) DGX_MIX(6)
-		default: return hipErrorInvalidValue;
+	MixRuns runs{};
+	int grid = 0;
+	for (int Nf = kHpMaxN; Nf >= 2; --Nf)
+		for (const MixRun& run : H.mruns) {
+			if (run.Nf != Nf || run.count == 0) continue;
+			if (runs.n == kHpMaxN) return hipErrorInvalidValue;   // one run per face-point count
+			const int i = runs.n++;
+			runs.Nf[i] = Nf;
+			runs.start[i] = run.start;
+			runs.count[i] = run.count;
+			runs.block0[i] = grid;
+			grid += (run.count + mix_fpb(Nf) - 1) / mix_fpb(Nf);
 		}
-#undef DGX_MIX
-		const hipError_t e = hipGetLastError();
-		if (e != hipSuccess) return e;
+	if (grid == 0) return hipSuccess;
+	const dim3 block(64 * kMixWaves);
+	if (ns) {
+		if (lf) hipLaunchKernelGGL((k_mix_faces<T, DGX_FLUX_LF, true>), dim3(grid), block, 0, c.stream, a, runs);
+		else hipLaunchKernelGGL((k_mix_faces<T, DGX_FLUX_ROE, true>), dim3(grid), block, 0, c.stream, a, runs);
+	} else {
+		if (lf) hipLaunchKernelGGL((k_mix_faces<T, DGX_FLUX_LF, false>), dim3(grid), block, 0, c.stream, a, runs);
+		else hipLaunchKernelGGL((k_mix_faces<T, DGX_FLUX_ROE, false>), dim3(grid), block, 0, c.stream, a, runs);
 	}
-	return hipSuccess;
+	return hipGetLastError();
 }
 
 }  // namespace
@@ -1484,14 +1525,9 @@ hipError_t launch_tri_minv64(const TriGroup& g, const TriOps<double>* ops, doubl
 #undef DGX_TRI_SWITCH
 #undef DGX_TRI_SWITCH_T
 
-hipError_t launch_mix_faces64(const HpData& H, const Ctx& c, const double* u, hipStream_t)
+hipError_t launch_mix_faces64(const HpData& H, const Ctx& c, const double* u, bool ns)
 {
-	return launch_mix(H, c, u, false);
-}
-
-hipError_t launch_mix_faces_ns64(const HpData& H, const Ctx& c, const double* u, hipStream_t)
-{
-	return launch_mix(H, c, u, true);
+	return launch_mix(H, c, u, ns);
 }
 
 hipError_t launch_mix_faces32(const HpData& H, const Ctx& c, const float* u, bool ns)
