@@ -178,13 +178,14 @@ __device__ inline void sweep_inplace2(S* buf, const R* M, int dir, int t)
 }
 
 // 2-D interpolation (I along a, then along b) of NB blocks of N x N values in place, one block per
-// thread (the last NB threads of the element), no barrier needed: each block is private to its thread.
-template <typename S, typename R, int N, int NB, int NT>
-__device__ inline void face_block_interp(S* buf, const R* M, int t)
+// thread, no barrier needed: each block is private to its thread.  The blocks of the workgroup's EPB elements (buf: the
+// first one's; STRIDE apart) go to its last EPB * NB threads, so that they fill whole wavefronts.
+template <typename S, typename R, int N, int NB, int NT, int EPB, int STRIDE>
+__device__ inline void face_block_interp(S* buf, const R* M, int tg)
 {
-	const int bi = t - (NT - NB);
+	const int bi = tg - EPB * (NT - NB);
 	if (bi < 0) return;
-	S* blk = buf + bi * N * N;
+	S* blk = buf + (bi / NB) * STRIDE + (bi % NB) * N * N;
 	S T[N][N];  // T[q][b] = sum_j M[q][j] blk[j + N b]
 #pragma unroll
 	for (int b = 0; b < N; ++b) {
@@ -302,14 +303,24 @@ __device__ inline void sweep_to_pb(const S* src, S* dst, const R* M, int base)
 	__syncthreads();
 }
 
-// Elements per workgroup: as many as fit 256 lanes and 56 KB of LDS, except HEX p=4 with float storage
-// (the FP32 and mixed residuals), where one element per workgroup measured 5% faster on 64^3 elements
-// (FP32 1.35 against 1.40 ms, mixed 1.73 against 1.82 ms, identical results); FP64 keeps two (2.45
-// against 2.74 ms).
-template <typename S, int D, int N, int NV>
+// Elements per workgroup: as many as fit 256 lanes and 56 KB of LDS, except where fewer measured faster (FP64, us):
+// * one wavefront where it is nearly full, QUAD p <= 3 and HEX p = 2: its barriers cost nothing and the LDS of a CU is used
+//   up in smaller pieces (HEX p = 2 32^3 91.7 -> 83.2, QUAD p = 1 300^2 30.0 -> 28.1, QUAD p = 3 128^2 14.9 -> 14.6);
+// * HEX p = 3: three elements, five workgroups a CU; four take 41 KB and leave three workgroups (32^3 200.8 -> 175.4);
+// * HEX p = 1: 24 elements took 56 KB and, with 258 registers, one wavefront a SIMD (40^3 220 -> 112);
+// * the forms with the limiter or a max-norm keep the full workgroups in these cases: each ends in global atomics (QUAD
+//   p = 3 128^2 RK3 with the limiter, 10 steps: 646 against 693); advection has no limiter and gains (16^2, 100 steps, 2547
+//   -> 2299);
+// * HEX p = 4 with float storage (FP32 and mixed): one element (64^3 mixed 1.61 ms against 1.66); FP64 keeps two (64^3 2.45 ms
+//   against 2.74).
+template <typename S, int D, int N, int NV, int MODE>
 constexpr int rhs_epb()
 {
+	constexpr bool norm = NV > 1 && (MODE == MODE_RHS_MINV || MODE == MODE_RK || MODE == MODE_RK_POS);
 	if (D == 3 && N == 5 && sizeof(S) == 4) return 1;
+	if (sizeof(S) == 8 && D == 3 && N == 4) return 3;
+	if (sizeof(S) == 8 && D == 3 && N <= 3 && !norm) return N == 3 ? 2 : 8;
+	if (sizeof(S) == 8 && D == 2 && N <= 4 && !norm) return 64 / (N * N);
 	constexpr int Np = ipow(N, D), NF = ipow(N, D - 1), NFACE = 2 * D;
 	constexpr int trsz = NFACE * NV * NF + (NFACE * NF > Np ? NFACE * NF : Np) * NV;
 	constexpr int bytes = (int)sizeof(S) * (NV * Np + trsz) + NFACE * 16;
@@ -335,7 +346,7 @@ __device__ inline void rhs_block_max(double m, unsigned long long* slot)
 }
 
 template <typename S, typename R, int D, int N, int PDE, int FLUX, int MODE>
-__global__ void __launch_bounds__(256) k_rhs(RhsArgs<S, R> a)
+__global__ void __launch_bounds__(256, D == 3 && N == 2 ? 2 : 1) k_rhs(RhsArgs<S, R> a)
 {
 #define DGX_RHS_PERSIST 0
 #include "k_rhs_body.inc"
@@ -357,7 +368,7 @@ template <typename S, typename R, int D, int N, int PDE, int FLUX, int MODE, boo
 inline hipError_t run_rhs(const RhsArgs<S, R>& a, hipStream_t st)
 {
 	constexpr int Np = ipow(N, D), NV = (PDE == DGX_PDE_EULER) ? D + 2 : 1;
-	constexpr int EPB = rhs_epb<S, D, N, NV>();
+	constexpr int EPB = rhs_epb<S, D, N, NV, MODE>();
 	const int grid = (((a.E + EPB - 1) / EPB) + 7) / 8 * 8;
 	if (a.E == 0) return hipSuccess;
 	if constexpr (PERSIST) {
