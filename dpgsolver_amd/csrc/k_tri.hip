@@ -17,9 +17,9 @@
 // M^-1 and the lift traces K_f = Ifc_f M^-1 tw0_f: the reference ones divided by det J on an affine group, each
 // element's own otherwise.
 //
-// Faces with a TRI side (k_mixf, k_mixf_ns): 2, 4 or 8 lanes per face (the next power of two >= Nf), four
+// Faces with a TRI side (k_mix_faces): 2, 4 or 8 lanes per face (the next power of two >= Nf), four
 // wavefronts per workgroup sharing one copy of the operators in LDS, each face's LDS steps synchronised within
-// its wavefront; one launch per face-point count Nf = max(p_L, p_R) + 1 (compute_face_reference_order,
+// its wavefront; one launch for all face-point counts Nf = max(p_L, p_R) + 1 (compute_face_reference_order,
 // face_solver.c:123-131; the faces arrive sorted by (Nf, types, orders), so a wavefront rarely mixes shapes).
 // The Navier-Stokes kernel forms the two sides' face gradients one after the other in the same LDS block, which
 // keeps its LDS per face at 16 Nf doubles.  Each side's own values
