@@ -252,13 +252,16 @@ dgx_status upload_uniform(dgx_ctx* h, const dgx_mesh* m, bool nonconf_ok)
 		const std::vector<double> hm = dgx::min_edge_lengths(d, c.N, c.E, m->xyz);
 		DGX_TRY(hipMalloc(&c.hmin, sizeof(double) * hm.size()));
 		DGX_TRY(hipMemcpy(c.hmin, hm.data(), sizeof(double) * hm.size(), hipMemcpyHostToDevice));
-		// greedy colouring of the face-neighbour graph (multicolour block Gauss-Seidel)
+		// greedy colouring of the face-neighbour graph (multicolour block Gauss-Seidel); an element that is its own
+		// neighbour has a coupling within its colour
+		c.self_neighbour = false;
 		std::vector<int> color(c.E, -1);
 		int ncol = 0;
 		for (int e = 0; e < c.E; ++e) {
 			unsigned used = 0;
 			for (int lf = 0; lf < NFACE; ++lf) {
 				const int n = ef[(size_t)e * NFACE + lf].en;
+				if (n == e) c.self_neighbour = true;
 				if (n >= 0 && n != e && color[n] >= 0 && color[n] < 32) used |= 1u << color[n];
 			}
 			int k = 0;

@@ -910,8 +910,9 @@ struct PrecondBlockSGS : Precond {
 	{
 		const size_t n = (size_t)c.E * c.Np * c.nv;
 		const int nc = (int)c.color_off.size() - 1;
-		// with two colours every neighbour of the first still holds zero: no face terms, nothing to clear
-		const bool two = nc == 2;
+		// with two colours every neighbour of the first still holds zero: no face terms, nothing to clear (not where an
+		// element is its own neighbour: the sweeps then read z within a colour too)
+		const bool two = nc == 2 && !c.self_neighbour;
 		if (!two)
 			DGX_HIP_CHECK(launch_fill_u64(c.stream, reinterpret_cast<unsigned long long*>(z), (int)n, 0ull));
 		for (int k = 0; k < nc; ++k) DGX_HIP_CHECK(run(c, k, v, false, (two && k == 0) ? 0 : -1, true, z, z, false));
@@ -919,7 +920,7 @@ struct PrecondBlockSGS : Precond {
 		for (int k = nc - 2; k >= 0; --k) DGX_HIP_CHECK(run(c, k, v, false, -1, true, z, z, false));
 		return hipSuccess;
 	}
-	// Two colours (1, 2), FP64 blocks.  The backward half-sweep leaves row 1 of A z = v exactly solved, so with
+	// Two colours (1, 2) without couplings inside a colour, FP64 blocks.  The backward half-sweep leaves row 1 of A z = v exactly solved, so with
 	// M = the sweeps' operator, A M^-1 is the identity on colour 1 and maps a vector that vanishes there to
 	//   v_2 + A_21 z_1,   z_1 = -A_11^-1 A_12 z_2,   z_2 = A_22^-1 v_2,
 	// which vanishes on colour 1 again.  Once the right-hand side is cleared on colour 1 (one block solve), the whole
@@ -929,7 +930,7 @@ struct PrecondBlockSGS : Precond {
 	// solves colour 2, then colour 1, leaves a residual on those nodes alone, and only the face-node rows of z_1 and
 	// z_2 are needed (k_pack_reduced).  QUAD p = 3: 105 MB of blocks an iteration on the 64 x 64 channel instead of the
 	// three sweeps' 235 MB and the product's traffic.
-	bool reducible(const Ctx& c) const override { return !fp32 && (int)c.color_off.size() == 3; }
+	bool reducible(const Ctx& c) const override { return !fp32 && (int)c.color_off.size() == 3 && !c.self_neighbour; }
 	static size_t count(const Ctx& c, int k) { return (size_t)(c.color_off[k + 1] - c.color_off[k]); }
 	static int rows(const Ctx& c) { return c.nv * (4 * c.N - 4); }
 	// the packed kernels' sizes: nv = 4, N <= 5 (the largest order that the in-LDS inverse takes)

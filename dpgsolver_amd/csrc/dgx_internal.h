@@ -213,6 +213,7 @@ struct Ctx {
 	double* hmin = nullptr;         // E: minimum straight edge length (compute_min_length_measure)
 	int* color_elems = nullptr;     // E: elements grouped by colour (no two face neighbours share a colour)
 	std::vector<int> color_off;     // n_colors + 1 offsets into color_elems
+	bool self_neighbour = false;    // some element meets itself across a periodic face (one element in that direction)
 	dgx_mlp* mlp = nullptr;         // attached learned preconditioner (not owned)
 	double* ns_gvt = nullptr;       // Navier-Stokes: face traces of the volume gradient (E x 2d x d x nv x Nfc)
 	double* ns_kappa = nullptr;     // Navier-Stokes: BR2 lift trace factor per face node (E x 2d x Nfc)
