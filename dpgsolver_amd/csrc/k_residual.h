@@ -93,9 +93,12 @@ __device__ inline int face_vol_node(int lf, int i)
 	return a + N * (b + N * fix);
 }
 
+// The sweeps are always inlined: as functions they take the operators by vector loads and hold a whole call's registers
+// (HEX linear operator p = 4 28^3 914 -> 387 us, p = 2 373 -> 117, p = 1 118 -> 52).
+//
 // In-place sweep along `dir` over NB blocks of N^DD values.
 template <typename S, typename R, int DD, int N, int NB, int NT>
-__device__ inline void sweep_inplace(S* buf, const R* M, int dir, int t)
+__device__ __forceinline__ void sweep_inplace(S* buf, const R* M, int dir, int t)
 {
 	constexpr int BL = ipow(N, DD);
 	constexpr int NL = ipow(N, DD - 1);
@@ -134,7 +137,7 @@ __device__ inline void sweep_inplace(S* buf, const R* M, int dir, int t)
 // Two independent in-place sweeps over one buffer: region A (NB1 blocks of N^D1 at offset 0) and
 // region B (NB2 blocks of N^D2 at offset OFFB), sharing one read / barrier / write / barrier cycle.
 template <typename S, typename R, int D1, int N, int NB1, int D2, int NB2, int OFFB, int NT>
-__device__ inline void sweep_inplace2(S* buf, const R* M, int dir, int t)
+__device__ __forceinline__ void sweep_inplace2(S* buf, const R* M, int dir, int t)
 {
 	constexpr int BL1 = ipow(N, D1), NL1 = ipow(N, D1 - 1), NP1 = NB1 * NL1;
 	constexpr int BL2 = ipow(N, D2), NL2 = ipow(N, D2 - 1), NP2 = NB2 * NL2;
@@ -181,7 +184,7 @@ __device__ inline void sweep_inplace2(S* buf, const R* M, int dir, int t)
 // thread, no barrier needed: each block is private to its thread.  The blocks of the workgroup's EPB elements (buf: the
 // first one's; STRIDE apart) go to its last EPB * NB threads, so that they fill whole wavefronts.
 template <typename S, typename R, int N, int NB, int NT, int EPB, int STRIDE>
-__device__ inline void face_block_interp(S* buf, const R* M, int tg)
+__device__ __forceinline__ void face_block_interp(S* buf, const R* M, int tg)
 {
 	const int bi = tg - EPB * (NT - NB);
 	if (bi < 0) return;
@@ -213,7 +216,7 @@ __device__ inline void face_block_interp(S* buf, const R* M, int tg)
 
 // dst (+)= sweep(src) along dir over NB blocks of N^DD values (src != dst).
 template <typename S, typename R, int DD, int N, int NB, int NT, bool ACC>
-__device__ inline void sweep_to(const S* src, S* dst, const R* M, int dir, int t)
+__device__ __forceinline__ void sweep_to(const S* src, S* dst, const R* M, int dir, int t)
 {
 	constexpr int BL = ipow(N, DD);
 	constexpr int NL = ipow(N, DD - 1);
@@ -256,7 +259,7 @@ __device__ inline int pencil_base(int pen, int dir)
 
 // in-place sweep along DIR of the thread's pencil (base < 0: idle thread, still takes both barriers)
 template <typename S, typename R, int N, int DIR>
-__device__ inline void sweep_inplace_pb(S* buf, const R* M, int base)
+__device__ __forceinline__ void sweep_inplace_pb(S* buf, const R* M, int base)
 {
 	constexpr int Sd = (DIR == 0) ? 1 : (DIR == 1 ? N : N * N);
 	S in[N];
@@ -279,7 +282,7 @@ __device__ inline void sweep_inplace_pb(S* buf, const R* M, int base)
 
 // dst (+)= sweep(src) along DIR for the thread's pencil (src != dst); the accumulation starts from dst
 template <typename S, typename R, int N, int DIR, bool ACC>
-__device__ inline void sweep_to_pb(const S* src, S* dst, const R* M, int base)
+__device__ __forceinline__ void sweep_to_pb(const S* src, S* dst, const R* M, int base)
 {
 	constexpr int Sd = (DIR == 0) ? 1 : (DIR == 1 ? N : N * N);
 	if (base >= 0) {
@@ -303,11 +306,14 @@ __device__ inline void sweep_to_pb(const S* src, S* dst, const R* M, int base)
 	__syncthreads();
 }
 
-// Elements per workgroup: as many as fit 256 lanes and 56 KB of LDS, except where fewer measured faster (FP64, us):
+// Elements per workgroup: as many as fit 256 lanes and 56 KB of LDS, except where fewer measured faster (us; FP64 unless
+// said):
 // * one wavefront where it is nearly full, QUAD p <= 3 and HEX p = 2: its barriers cost nothing and the LDS of a CU is used
-//   up in smaller pieces (HEX p = 2 32^3 91.7 -> 83.2, QUAD p = 1 300^2 30.0 -> 28.1, QUAD p = 3 128^2 14.9 -> 14.6);
+//   up in smaller pieces (HEX p = 2 32^3 91.7 -> 83.2, QUAD p = 1 300^2 30.0 -> 28.1, QUAD p = 3 128^2 14.9 -> 14.6;
+//   FP32 and mixed HEX p = 2 8^3 12.4 -> 10.6 and 13.8 -> 11.7, linear operator 28^3 373 -> 117 with inlined sweeps);
 // * HEX p = 3: three elements, five workgroups a CU; four take 41 KB and leave three workgroups (32^3 200.8 -> 175.4);
-// * HEX p = 1: 24 elements took 56 KB and, with 258 registers, one wavefront a SIMD (40^3 220 -> 112);
+// * HEX p = 1: 24 elements took 56 KB and, with 258 registers, one wavefront a SIMD (40^3 220 -> 112; FP32 had 32 elements
+//   in 39 KB, mixed in 44);
 // * the forms with the limiter or a max-norm keep the full workgroups in these cases: each ends in global atomics (QUAD
 //   p = 3 128^2 RK3 with the limiter, 10 steps: 646 against 693); advection has no limiter and gains (16^2, 100 steps, 2547
 //   -> 2299);
@@ -319,7 +325,7 @@ constexpr int rhs_epb()
 	constexpr bool norm = NV > 1 && (MODE == MODE_RHS_MINV || MODE == MODE_RK || MODE == MODE_RK_POS);
 	if (D == 3 && N == 5 && sizeof(S) == 4) return 1;
 	if (sizeof(S) == 8 && D == 3 && N == 4) return 3;
-	if (sizeof(S) == 8 && D == 3 && N <= 3 && !norm) return N == 3 ? 2 : 8;
+	if (D == 3 && N <= 3 && !norm) return N == 3 ? 2 : 8;
 	if (sizeof(S) == 8 && D == 2 && N <= 4 && !norm) return 64 / (N * N);
 	constexpr int Np = ipow(N, D), NF = ipow(N, D - 1), NFACE = 2 * D;
 	constexpr int trsz = NFACE * NV * NF + (NFACE * NF > Np ? NFACE * NF : Np) * NV;
@@ -345,8 +351,10 @@ __device__ inline void rhs_block_max(double m, unsigned long long* slot)
 	if ((int)(threadIdx.x & 63) == __builtin_ctzll(act)) atomicMax(slot, b);
 }
 
+// HEX p = 1 in FP64 alone is held to two wavefronts a SIMD (M^-1 R 32^3 145 -> 101 us); dual numbers spill there (linear
+// operator 28^3 99 -> 118), FP32 fits without.
 template <typename S, typename R, int D, int N, int PDE, int FLUX, int MODE>
-__global__ void __launch_bounds__(256, D == 3 && N == 2 ? 2 : 1) k_rhs(RhsArgs<S, R> a)
+__global__ void __launch_bounds__(256, D == 3 && N == 2 && sizeof(S) == 8 ? 2 : 1) k_rhs(RhsArgs<S, R> a)
 {
 #define DGX_RHS_PERSIST 0
 #include "k_rhs_body.inc"
