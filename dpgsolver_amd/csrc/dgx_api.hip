@@ -59,6 +59,11 @@ void free_hp(Ctx& c)
 	}
 	release(H->tri_ops64); release(H->tri_ops32); release(H->mfaces); release(H->mnJ); release(H->mnJ32);
 	release(H->mxy);
+	for (int k = 0; k < dgx::HpData::kLanes; ++k) {
+		if (H->lane[k]) (void)hipStreamDestroy(H->lane[k]);
+		if (H->join_ev[k]) (void)hipEventDestroy(H->join_ev[k]);
+	}
+	if (H->fork_ev) (void)hipEventDestroy(H->fork_ev);
 	delete H;
 	c.hp = nullptr;
 }
@@ -390,9 +395,9 @@ void outward_nj(const double* xyz, int N, int lf, const double* s, int ns, doubl
 	}
 }
 
-// Enqueues launch(g, s) for every order group on the caller's stream.  Each group context gets its own stream back
-// afterwards (during a graph capture the caller's is the private capture stream, destroyed when the capture ends, and a
-// group context must never keep it).
+// Enqueues launch(g, s) for every order group, on the caller's stream or between fork and join on the group's side stream.
+// Each group context gets its own stream back afterwards (during a graph capture the caller's is the private capture
+// stream, destroyed when the capture ends, and a group context must never keep it).
 template <typename F>
 hipError_t on_groups(Ctx& c, F launch)
 {
@@ -400,7 +405,7 @@ hipError_t on_groups(Ctx& c, F launch)
 	for (size_t g = 0; g < H.groups.size(); ++g) {
 		Ctx& s = H.groups[g]->c;
 		const hipStream_t own = s.stream;
-		s.stream = c.stream;
+		s.stream = H.forked ? H.lane[H.group_lane[g]] : c.stream;
 		const hipError_t e = launch(g, s);
 		s.stream = own;
 		if (e != hipSuccess) return e;
@@ -411,90 +416,149 @@ hipError_t on_groups(Ctx& c, F launch)
 // whether no face joins two orders or types: then no kernel between the groups reads gradient traces
 bool ns_groups_alone(const dgx::HpData& H) { return H.tri.empty() && H.Fnc == 0; }
 
+// Enqueues launch(t, stream) for every TRI group likewise.
+template <typename F>
+hipError_t on_tri_groups(Ctx& c, F launch)
+{
+	dgx::HpData& H = *c.hp;
+	for (size_t t = 0; t < H.tri.size(); ++t) DGX_HIP_CHECK(launch(t, H.forked ? H.lane[H.tri_lane[t]] : c.stream));
+	return hipSuccess;
+}
+
+// Whether a residual call spreads the launches of each phase over the side streams: while a graph is captured, and where
+// the launches are long enough.  The forks and joins cost an eager call 41 us a phase, more than the kernels gain side by
+// side; a replayed graph needs 140 us (Euler) or 170 (Navier-Stokes) for its branches however small the mesh.  Orders 1..5,
+// us a replay (waited for), one stream | side streams:
+//   Euler QUAD FP64          70 x 50 116 (138) | 146 (139)   120 x 90 148 (166) | 146 (137)   500 x 300 316 (329) | 244 (263)
+//   Euler QUAD FP32          120 x 90 114 (136) | 144 (137)  220 x 150 149 (167) | 146 (138)  500 x 300 216 (229) | 160 (178)
+//   Euler TRI / QUAD FP64    120 x 90 111 (122) | 124 (115)  220 x 150 134 (145) | 138 (135)  500 x 300 309 (321) | 303 (301)
+//   Navier-Stokes QUAD FP64  8 x 8 178 (191) | 174 (168)     120 x 90 253 (266) | 183 (197)   500 x 300 709 (720) | 579 (577)
+//   Navier-Stokes QUAD FP32  8 x 8 147 (161) | 175 (164)     70 x 50 169 (186) | 174 (170)    500 x 300 448 (460) | 344 (341)
+//   Navier-Stokes TRI / QUAD 8 x 8 136 (149) | 146 (143)     24 x 16 149 (162) | 145 (156)    500 x 300 806 (817) | 740 (738)
+bool hp_split(const Ctx& c, bool fp32)
+{
+	hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+	if (!c.stream || hipStreamIsCapturing(c.stream, &st) != hipSuccess || st != hipStreamCaptureStatusActive) return false;
+	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) return c.hp->E >= 256;
+	return c.hp->E >= (fp32 || !c.hp->tri.empty() ? 20000 : 10000);
+}
+
+// The phases of one residual call: fork at the start and after each barrier, join at each barrier and at the end, also where
+// a launch fails (an unjoined side stream would leave the capture open).
+struct HpPhases {
+	Ctx& c;
+	HpPhases(Ctx& c_, bool fp32) : c(c_)
+	{
+		c.hp->split = hp_split(c, fp32);
+		c.hp->forked = false;
+	}
+	~HpPhases() { (void)dgx::hp_join(c); }
+	hipError_t fork() { return dgx::hp_fork(c); }
+	hipError_t join() { return dgx::hp_join(c); }
+	hipError_t barrier()
+	{
+		const hipError_t e = dgx::hp_join(c);
+		return e != hipSuccess ? e : dgx::hp_fork(c);
+	}
+};
+
 // Variable-order and mixed-type residuals (FP64). Navier-Stokes: every group's gradient traces (TRI: and state
 // traces), the faces between orders or types (lifted gradients and fluxes; one launch per face-point count),
 // every group's residual (+ M^-1 and max-norm). Euler: the TRI state traces, the faces, every group's residual.
-// All on one stream: spread over side streams, the independent launches of a phase ran side by side, but each phase
-// paid a fork and a join over the streams, 41 us, and the kernels of all but the smallest groups fill the chip alone.
-// TRI / QUAD mesh with orders 1..5, FP64, four side streams against one, us: Euler 8 x 8 274 / 97, 300 x 200 293 / 179,
-// 500 x 300 378 / 331; Navier-Stokes 287 / 182, 447 / 436, 852 / 857 (before the faces of one phase became one launch).
+// Eager calls run on one stream, captured ones may split (hp_split).  Eager, TRI / QUAD mesh with orders 1..5, FP64, four
+// side streams against one, us: Euler 8 x 8 274 / 97, 300 x 200 293 / 179, 500 x 300 378 / 331; Navier-Stokes 287 / 182,
+// 447 / 436, 852 / 857 (before the faces of one phase became one launch).
 dgx_status hp_rhs64(Ctx& c, const double* u, double* r, int mode, unsigned long long* dmax)
 {
 	dgx::HpData& H = *c.hp;
 	if (!H.tri.empty() && mode != dgx::MODE_RHS && mode != dgx::MODE_RHS_MINV) return DGX_ERR_UNSUPPORTED;
 	const bool minv = (mode == dgx::MODE_RHS_MINV);
+	const bool tri = !H.tri.empty();
+	HpPhases ph(c, false);
+	DGX_TRY(ph.fork());
 	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		const double mu = c.cfg.mu, Pr = c.cfg.Pr;
 		// no faces between orders or types: each group's whole residual, as on a mesh of its order alone
 		const bool alone = ns_groups_alone(H);
-		auto residual = [&](size_t g, Ctx& s) -> hipError_t {
+		if (!alone) {
+			DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
+			DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+				return dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 1, s);
+			}));
+			DGX_TRY(tri ? ph.join() : ph.barrier());
+			DGX_TRY(tri ? dgx::launch_mix_faces64(H, c, u, true) : dgx::launch_hp_faces64(c, u));
+			DGX_TRY(ph.barrier());
+			DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+				const hipError_t e = dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 2, s);
+				return e == hipSuccess && minv ? dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, s) : e;
+			}));
+		}
+		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) -> hipError_t {
 			double* rg = r + H.u_off[g];
 			hipError_t e = dgx::launch_rhs_ns_phase(s, u + H.u_off[g], rg, alone ? 0 : 2);
-			if (e != hipSuccess || mode != dgx::MODE_RHS_MINV) return e;
+			if (e != hipSuccess || !minv) return e;
 			e = dgx::launch_minv(s, rg);
 			if (e == hipSuccess && dmax) e = dgx::launch_maxabs(s, rg, ndof(s), dmax);
 			return e;
-		};
-		if (alone) {
-			DGX_TRY(on_groups(c, residual));
-			return DGX_OK;
-		}
-		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
-		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 1, c.stream));
-		if (H.tri.empty()) DGX_TRY(dgx::launch_hp_faces64(c, u));
-		else DGX_TRY(dgx::launch_mix_faces64(H, c, u, true));
-		for (size_t t = 0; t < H.tri.size(); ++t) {
-			DGX_TRY(dgx::launch_tri_ns_phase64(H.tri[t], H.tri_ops64, u, r, H.z64, mu, Pr, 2, c.stream));
-			if (minv) DGX_TRY(dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, c.stream));
-		}
-		DGX_TRY(on_groups(c, residual));
+		}));
 	} else {
-		if (H.tri.empty()) {
-			DGX_TRY(dgx::launch_hp_faces64(c, u));
-		} else {   // the TRI traces, then the faces
-			for (size_t t = 0; t < H.tri.size(); ++t)
-				DGX_TRY(dgx::launch_tri_trace64(H.tri[t], H.tri_ops64, u, c.stream));
-			DGX_TRY(dgx::launch_mix_faces64(H, c, u, false));
+		if (tri) {   // the TRI traces, then the faces
+			DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+				return dgx::launch_tri_trace64(H.tri[t], H.tri_ops64, u, s);
+			}));
+			DGX_TRY(ph.join());
 		}
+		DGX_TRY(tri ? dgx::launch_mix_faces64(H, c, u, false) : dgx::launch_hp_faces64(c, u));
+		DGX_TRY(ph.barrier());
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs64(s, u + H.u_off[g], r + H.u_off[g], mode, dmax); }));
-		for (size_t t = 0; t < H.tri.size(); ++t) {
-			DGX_TRY(dgx::launch_tri_rhs64(H.tri[t], H.tri_ops64, u, r, H.z64, c.stream));
-			if (minv) DGX_TRY(dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, c.stream));
-		}
+		DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+			const hipError_t e = dgx::launch_tri_rhs64(H.tri[t], H.tri_ops64, u, r, H.z64, s);
+			return e == hipSuccess && minv ? dgx::launch_tri_minv64(H.tri[t], H.tri_ops64, r, dmax, s) : e;
+		}));
 	}
+	DGX_TRY(ph.join());
 	return DGX_OK;
 }
 
 dgx_status hp_rhs32(Ctx& c, const float* u, float* r)
 {
 	dgx::HpData& H = *c.hp;
+	const bool tri = !H.tri.empty();
+	HpPhases ph(c, true);
+	DGX_TRY(ph.fork());
 	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
 		const double mu = c.cfg.mu, Pr = c.cfg.Pr;
-		if (ns_groups_alone(H)) {
-			DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 0); }));
-			return DGX_OK;
+		const bool alone = ns_groups_alone(H);
+		if (!alone) {
+			DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
+			DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+				return dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 1, s);
+			}));
+			DGX_TRY(tri ? ph.join() : ph.barrier());
+			DGX_TRY(tri ? dgx::launch_mix_faces32(H, c, u, true) : dgx::launch_hp_faces32(c, u));
+			DGX_TRY(ph.barrier());
+			DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+				return dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 2, s);
+			}));
 		}
-		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
-		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 1, c.stream));
-		if (H.tri.empty()) DGX_TRY(dgx::launch_hp_faces32(c, u));
-		else DGX_TRY(dgx::launch_mix_faces32(H, c, u, true));
-		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_ns_phase32(H.tri[t], H.tri_ops32, u, r, H.z32, mu, Pr, 2, c.stream));
-		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], 2); }));
+		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) {
+			return dgx::launch_rhs_ns32_phase(s, u + H.u_off[g], r + H.u_off[g], alone ? 0 : 2);
+		}));
 	} else {
-		if (H.tri.empty()) {
-			DGX_TRY(dgx::launch_hp_faces32(c, u));
-		} else {   // the TRI traces, then the faces
-			for (size_t t = 0; t < H.tri.size(); ++t)
-				DGX_TRY(dgx::launch_tri_trace32(H.tri[t], H.tri_ops32, u, c.stream));
-			DGX_TRY(dgx::launch_mix_faces32(H, c, u, false));
+		if (tri) {   // the TRI traces, then the faces
+			DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+				return dgx::launch_tri_trace32(H.tri[t], H.tri_ops32, u, s);
+			}));
+			DGX_TRY(ph.join());
 		}
+		DGX_TRY(tri ? dgx::launch_mix_faces32(H, c, u, false) : dgx::launch_hp_faces32(c, u));
+		DGX_TRY(ph.barrier());
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs32(s, u + H.u_off[g], r + H.u_off[g]); }));
-		for (size_t t = 0; t < H.tri.size(); ++t)
-			DGX_TRY(dgx::launch_tri_rhs32(H.tri[t], H.tri_ops32, u, r, H.z32, c.stream));
+		DGX_TRY(on_tri_groups(c, [&](size_t t, hipStream_t s) {
+			return dgx::launch_tri_rhs32(H.tri[t], H.tri_ops32, u, r, H.z32, s);
+		}));
 	}
+	DGX_TRY(ph.join());
 	return DGX_OK;
 }
 
@@ -503,16 +567,25 @@ dgx_status hp_rhs_mixed(Ctx& c, const double* u, float* r)
 {
 	dgx::HpData& H = *c.hp;
 	if (!H.tri.empty()) return DGX_ERR_UNSUPPORTED;   // TRI elements: FP64 only
-	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES && ns_groups_alone(H)) {
-		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 0); }));
-	} else if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
-		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
-		DGX_TRY(dgx::launch_hp_faces_mixed(c, u));
-		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 2); }));
+	HpPhases ph(c, false);
+	DGX_TRY(ph.fork());
+	if (c.cfg.pde == DGX_PDE_NAVIER_STOKES) {
+		const bool alone = ns_groups_alone(H);
+		if (!alone) {
+			DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], 1); }));
+			DGX_TRY(ph.barrier());
+			DGX_TRY(dgx::launch_hp_faces_mixed(c, u));
+			DGX_TRY(ph.barrier());
+		}
+		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) {
+			return dgx::launch_rhs_ns_mixed_phase(s, u + H.u_off[g], r + H.u_off[g], alone ? 0 : 2);
+		}));
 	} else {
 		DGX_TRY(dgx::launch_hp_faces_mixed(c, u));
+		DGX_TRY(ph.barrier());
 		DGX_TRY(on_groups(c, [&](size_t g, Ctx& s) { return dgx::launch_rhs_mixed(s, u + H.u_off[g], r + H.u_off[g]); }));
 	}
+	DGX_TRY(ph.join());
 	return DGX_OK;
 }
 
@@ -974,6 +1047,42 @@ static dgx_status upload_hp_impl(dgx_ctx* h, int E, int F, const int* type, cons
 		sub->c.hp_z64 = H.z64 + H.z_off[g];
 		sub->c.hp_z32 = H.z32 + H.z_off[g];
 	}
+	// side streams, and the groups and face pairs spread over them longest first (cost ~ items x N^2)
+	for (int k = 0; k < dgx::HpData::kLanes; ++k) {
+		DGX_TRY(hipStreamCreateWithFlags(&H.lane[k], hipStreamNonBlocking));
+		DGX_TRY(hipEventCreateWithFlags(&H.join_ev[k], hipEventDisableTiming));
+	}
+	DGX_TRY(hipEventCreateWithFlags(&H.fork_ev, hipEventDisableTiming));
+	auto balance = [](const std::vector<double>& cost) {
+		std::vector<int> idx(cost.size()), lane(cost.size(), 0);
+		for (size_t i = 0; i < idx.size(); ++i) idx[i] = (int)i;
+		std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return cost[a] > cost[b]; });
+		double load[dgx::HpData::kLanes] = {};
+		for (int i : idx) {
+			int k = 0;
+			for (int j = 1; j < dgx::HpData::kLanes; ++j)
+				if (load[j] < load[k]) k = j;
+			lane[i] = k;
+			load[k] += cost[i];
+		}
+		return lane;
+	};
+	// the QUAD and TRI groups of one phase share the streams: one balance over both (a TRI element's dense
+	// products cost about Np Nc / 3 against N^2 per QUAD element, from the measured kernel times)
+	std::vector<double> gcost(G + T), pcost(H.pairs.size());
+	for (int g = 0; g < G; ++g) gcost[g] = (double)(e_off[g + 1] - e_off[g]) * (order[g] + 1) * (order[g] + 1);
+	for (int t = 0; t < T; ++t) {
+		const int p = tri_p[t], np = (p + 1) * (p + 2) / 2, nc = p == 1 ? 3 : p == 2 ? 6 : p == 3 ? 12 : p == 4 ? 16 : 25;
+		gcost[G + t] = (double)(tri_e0[t + 1] - tri_e0[t]) * np * nc / 3.0;
+	}
+	for (size_t i = 0; i < H.pairs.size(); ++i) {
+		const int n = std::max(H.pairs[i].NL, H.pairs[i].NR);
+		pcost[i] = (double)H.pairs[i].count * n * n;
+	}
+	const std::vector<int> lanes = balance(gcost);
+	H.group_lane.assign(lanes.begin(), lanes.begin() + G);
+	H.tri_lane.assign(lanes.begin() + G, lanes.end());
+	H.pair_lane = balance(pcost);
 	H.ready = true;
 	return DGX_OK;
 }

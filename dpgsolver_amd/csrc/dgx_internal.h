@@ -177,6 +177,16 @@ struct HpData {
 	float* z32 = nullptr;
 	HpOps<double>* ops64 = nullptr;
 	HpOps<float>* ops32 = nullptr;
+	// Side streams (default priority) over which the independent launches of one phase are spread while a graph is
+	// captured (see hp_split): they write disjoint outputs, so they run concurrently between a fork (each side stream
+	// waits for the capturing stream) and a join.
+	static constexpr int kLanes = 4;
+	hipStream_t lane[kLanes] = {};
+	hipEvent_t fork_ev = nullptr;
+	hipEvent_t join_ev[kLanes] = {};
+	bool split = false, forked = false;    // this call splits its phases; the side streams are between fork and join
+	std::vector<int> group_lane, tri_lane; // side stream of each group (one longest-first balance of both kinds' costs)
+	std::vector<int> pair_lane;            // and of each face pair
 	// TRI groups and the faces that touch a TRI element (mixed meshes)
 	std::vector<TriGroup> tri;
 	TriOps<double>* tri_ops64 = nullptr;   // device: kTriMaxP + 1 entries, indexed by p
@@ -189,6 +199,10 @@ struct HpData {
 	std::vector<MixRun> mruns;             // runs of mixed faces with one Nf
 };
 
+struct Ctx;
+// Fork and join of the side streams around one phase (nothing where the call does not split).
+hipError_t hp_fork(Ctx& c);
+hipError_t hp_join(Ctx& c);
 
 // Per-element face record: f, neighbour element (-1 on a boundary), and packed
 // (neighbour local face | side << 4 | ord << 8 | bc << 12).

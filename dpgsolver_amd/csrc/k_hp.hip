@@ -403,7 +403,7 @@ hipError_t run_hp_faces(Ctx& c, const S* u, const double* u64, S* z, const S* nJ
 		const bool lf = c.cfg.num_flux == DGX_FLUX_LF;
 		for (size_t ip = 0; ip < H.pairs.size(); ++ip) {
 			const HpPair& pr = H.pairs[ip];
-			const hipStream_t st = c.stream;
+			const hipStream_t st = H.forked ? H.lane[H.pair_lane[ip]] : c.stream;
 			const int blocks = (pr.count + 7) / 8;
 #define DGX_HP_PAIR(L, R)                                                                                              \
 	case L * 8 + R:                                                                                                    \
@@ -427,7 +427,7 @@ hipError_t run_hp_faces(Ctx& c, const S* u, const double* u64, S* z, const S* nJ
 	const bool lf = c.cfg.num_flux == DGX_FLUX_LF;
 	for (size_t ip = 0; ip < H.pairs.size(); ++ip) {
 		const HpPair& pr = H.pairs[ip];
-		const hipStream_t st = c.stream;
+		const hipStream_t st = H.forked ? H.lane[H.pair_lane[ip]] : c.stream;
 		const int blocks = (pr.count + 7) / 8;
 #define DGX_HP_PAIR(L, R)                                                                                              \
 	case L * 8 + R:                                                                                                    \
@@ -449,6 +449,31 @@ hipError_t run_hp_faces(Ctx& c, const S* u, const double* u64, S* z, const S* nJ
 }
 
 }  // namespace
+
+// Both run inside graph captures, so each event is recorded on this call, in the current capture, before any stream waits
+// on it: a wait on an event whose last record belonged to an earlier capture (whose graph may since have been destroyed)
+// would make the capture depend on nodes of that other graph.
+hipError_t hp_fork(Ctx& c)
+{
+	HpData& H = *c.hp;
+	if (!H.split) return hipSuccess;
+	H.forked = true;
+	DGX_HIP_CHECK(hipEventRecord(H.fork_ev, c.stream));
+	for (int k = 0; k < HpData::kLanes; ++k) DGX_HIP_CHECK(hipStreamWaitEvent(H.lane[k], H.fork_ev, 0));
+	return hipSuccess;
+}
+
+hipError_t hp_join(Ctx& c)
+{
+	HpData& H = *c.hp;
+	if (!H.forked) return hipSuccess;
+	H.forked = false;
+	for (int k = 0; k < HpData::kLanes; ++k) {
+		DGX_HIP_CHECK(hipEventRecord(H.join_ev[k], H.lane[k]));
+		DGX_HIP_CHECK(hipStreamWaitEvent(c.stream, H.join_ev[k], 0));
+	}
+	return hipSuccess;
+}
 
 // The face kernels between orders, one launch per (NL, NR) pair.
 hipError_t launch_hp_faces64(Ctx& c, const double* u)

@@ -347,10 +347,10 @@ def test_hp_graph_replays_equal_eager_calls(dev):
 
 
 def test_hp_residual_on_a_caller_stream(dev):
-    """A variable-order residual spreads its launches over the context's side streams and joins them back to the
-    caller's stream: on a caller stream other than the default one, work enqueued on that stream right after
-    the call (a copy of the residual) sees the whole residual, eagerly and through a graph, bitwise equal to
-    the same call on the default stream."""
+    """A variable-order residual enqueues all its launches on the caller's stream (a captured one may fork them over the
+    context's side streams and joins them back): on a caller stream other than the default one, work enqueued on that
+    stream right after the call (a copy of the residual) sees the whole residual, eagerly and through a graph, bitwise
+    equal to the same call on the default stream."""
     from dpgsolver_amd import _lib
 
     n = (6, 5)
