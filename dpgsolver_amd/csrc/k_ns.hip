@@ -244,8 +244,13 @@ __global__ void __launch_bounds__(128) k_ns_gv(NsArgs<S> a)
 // once instead of twice.  448 x 448, Roe, FP64: 306 -> 242 us (222 here: the FP64 pipe takes 138, LDS 122 of them).
 // LDS regions change hands: the face traces (own and neighbour) become the face products in place, the volume gradient
 // becomes the weighted fluxes, the GLL state becomes the face fluxes.
+// The mixed form (PERT) keeps the halves in FP64, as its face fluxes are: rounded to FP32 on their way they added to the
+// error of the residual (against FP64, p = 1..5, 12^2 .. 200^2, geometric mean 1.0033 of the gradient-trace kernels' error;
+// now 0.9992; 448 x 448 p = 3 215 us there, 183 with FP32 halves, 198).
+template <bool PERT, typename S> struct NsHalf { using type = S; };
+template <typename S> struct NsHalf<true, S> { using type = double; };
 template <typename S, int N, int FLUX, bool PERT, bool SUTH>
-__global__ void __launch_bounds__(128) k_ns_own(NsArgs<S> a, S* __restrict__ half)
+__global__ void __launch_bounds__(128) k_ns_own(NsArgs<S> a, typename NsHalf<PERT, S>::type* __restrict__ half)
 {
 	using G = typename NsArgs<S>::G;
 	constexpr int Np = N * N, EPB = ns_epb<S, N>(), TS = 4 * kNsNV * N;
@@ -366,7 +371,7 @@ __global__ void __launch_bounds__(128) k_ns_own(NsArgs<S> a, S* __restrict__ hal
 			gf[kNsNV + v] += eta * kap * q1;
 		}
 		const S sgn = side == 0 ? S(1.0) : S(-1.0);
-		S hv[kNsNV];   // J_f n . fv / 2 of the own side
+		typename NsHalf<PERT, S>::type hv[kNsNV];   // J_f n . fv / 2 of the own side
 		if constexpr (PERT) {
 			// FP64 states c_e + delta and fluxes; the normal Euler flux of c_e is subtracted before rounding
 			const double* ce = B.C[slc];
@@ -394,7 +399,7 @@ __global__ void __launch_bounds__(128) k_ns_own(NsArgs<S> a, S* __restrict__ hal
 #pragma unroll
 			for (int v = 0; v < kNsNV; ++v) {
 				double vis = 0.5 * (nd[0] * fv[0 + 2 * v] + nd[1] * fv[1 + 2 * v]);
-				hv[v] = S(vis * Jd);
+				hv[v] = vis * Jd;
 				if (wall) vis += 0.5 * (nd[0] * fw[0 + 2 * v] + nd[1] * fw[1 + 2 * v]);
 				// no-slip flux walls: the energy flux is the provided one (numerical_flux_central_T.c:222-230)
 				const double tot = (nf_provided && v == kNsNV - 1) ? a.walls.nfE : fdn[v] + vis;
@@ -419,7 +424,7 @@ __global__ void __launch_bounds__(128) k_ns_own(NsArgs<S> a, S* __restrict__ hal
 		}
 		// the other side tests with the opposite sign
 #pragma unroll
-		for (int v = 1; v < kNsNV; ++v) half[(((size_t)e * 4 + lf) * 3 + v - 1) * N + o] = -sgn * hv[v];
+		for (int v = 1; v < kNsNV; ++v) half[(((size_t)e * 4 + lf) * 3 + v - 1) * N + o] = side == 0 ? -hv[v] : hv[v];
 	}
 	__syncthreads();   // face products and fluxes are complete, the gradient traces taken
 	if (valid) {
@@ -505,22 +510,25 @@ __global__ void __launch_bounds__(128) k_ns_own(NsArgs<S> a, S* __restrict__ hal
 	if (valid)
 #pragma unroll
 		for (int v = 0; v < kNsNV; ++v) {
-			S acc = S(0.0);
+			// (PERT: summed in FP64, since k_ns_add rounds the residual once more)
+			using H = typename NsHalf<PERT, S>::type;
+			H acc = H(0.0);
 #pragma unroll
-			for (int mm = 0; mm < N; ++mm) acc += B.I[mm * N + c0] * GX[slc][v * Np + mm + N * c1];
-			a.out[((size_t)e * kNsNV + v) * Np + t] = acc;
+			for (int mm = 0; mm < N; ++mm) acc += H(B.I[mm * N + c0]) * H(GX[slc][v * Np + mm + N * c1]);
+			a.out[((size_t)e * kNsNV + v) * Np + t] = S(acc);
 		}
 }
 
 // r -= the neighbours' viscous halves, lifted onto the face nodes: sum_a I[a][b] w_a half(a) at node b of the face.
 // Bound by memory, 47 us at 448 x 448, p = 3 (1.1 KB an element).  Halves to LDS first, one face point per lane: gathered
 // by every lane of a face they took 142 us of address work.
-template <typename S, int N>
-__global__ void __launch_bounds__(256) k_ns_add(const ElemFace* __restrict__ ef, const Ops1D<S>* __restrict__ ops,
-                                                const S* __restrict__ half, S* __restrict__ r, int E)
+// H: the halves' type, in which they are lifted too.
+template <typename S, typename H, int N>
+__global__ void __launch_bounds__(256) k_ns_add(const ElemFace* __restrict__ ef, const Ops1D<H>* __restrict__ ops,
+                                                const H* __restrict__ half, S* __restrict__ r, int E)
 {
 	constexpr int Np = N * N, EPB = 256 / Np;
-	__shared__ S sIw[Np], sh[EPB][4][3][N];   // I[a][b] w_a; the neighbours' halves, own ordering
+	__shared__ H sIw[Np], sh[EPB][4][3][N];   // I[a][b] w_a; the neighbours' halves, own ordering
 	const int sl = threadIdx.x / Np, t = threadIdx.x % Np, e = blockIdx.x * EPB + sl;
 	const bool valid = sl < EPB && e < E;
 	for (int i = threadIdx.x; i < Np; i += 256) sIw[i] = ops->I[i] * ops->w[i / N];
@@ -531,12 +539,12 @@ __global__ void __launch_bounds__(256) k_ns_add(const ElemFace* __restrict__ ef,
 			const int q = ((f.packed >> 8) & 7) ? N - 1 - o : o;   // 2-D: the orientation bits are 0 or 2 (reversed)
 #pragma unroll
 			for (int v = 0; v < 3; ++v)
-				sh[sl][lf][v][o] = f.en >= 0 ? half[(((size_t)f.en * 4 + (f.packed & 15)) * 3 + v) * N + q] : S(0.0);
+				sh[sl][lf][v][o] = f.en >= 0 ? half[(((size_t)f.en * 4 + (f.packed & 15)) * 3 + v) * N + q] : H(0.0);
 		}
 	__syncthreads();
 	const int c0 = t % N, c1 = t / N;
 	if (!valid || (c0 != 0 && c0 != N - 1 && c1 != 0 && c1 != N - 1)) return;
-	S acc[3] = {};
+	H acc[3] = {};
 #pragma unroll
 	for (int lf = 0; lf < 4; ++lf) {
 		const int fd = lf >> 1;
@@ -548,7 +556,10 @@ __global__ void __launch_bounds__(256) k_ns_add(const ElemFace* __restrict__ ef,
 			for (int v = 0; v < 3; ++v) acc[v] += sIw[q * N + b] * sh[sl][lf][v][q];
 	}
 #pragma unroll
-	for (int v = 0; v < 3; ++v) r[((size_t)e * kNsNV + 1 + v) * Np + t] -= acc[v];
+	for (int v = 0; v < 3; ++v) {
+		S& x = r[((size_t)e * kNsNV + 1 + v) * Np + t];
+		x = S(H(x) - acc[v]);
+	}
 }
 
 template <typename S, int N, int FLUX, bool PERT, int MODE, bool SUTH>
@@ -897,7 +908,11 @@ hipError_t run_ns(Ctx& c, const NsArgs<S>& a, int phase)
 	if constexpr (MODE == kNsRhs) {
 		if (phase == 0) {   // one order, no faces between orders: the gradient-trace buffer holds the viscous halves
 			const bool lf = c.cfg.num_flux == DGX_FLUX_LF;
-			S* half = a.gvt;
+			using H = typename NsHalf<PERT, S>::type;
+			H* half = reinterpret_cast<H*>(a.gvt);   // 12 N values an element of the buffer's 32 N doubles
+			const Ops1D<H>* ops;
+			if constexpr (PERT) ops = c.ops64;
+			else ops = a.ops;
 #define DGX_NS_OWN(FL, SU) hipLaunchKernelGGL((k_ns_own<S, N, FL, PERT, SU>), dim3(grid), dim3(EPB * Np), 0, c.stream, a, half)
 			if (a.sutherland) {
 				if (lf) DGX_NS_OWN(DGX_FLUX_LF, true);
@@ -909,7 +924,7 @@ hipError_t run_ns(Ctx& c, const NsArgs<S>& a, int phase)
 #undef DGX_NS_OWN
 			DGX_HIP_CHECK(hipGetLastError());
 			constexpr int AEPB = 256 / Np;
-			hipLaunchKernelGGL((k_ns_add<S, N>), dim3((c.E + AEPB - 1) / AEPB), dim3(256), 0, c.stream, c.elem_faces, a.ops, half,
+			hipLaunchKernelGGL((k_ns_add<S, H, N>), dim3((c.E + AEPB - 1) / AEPB), dim3(256), 0, c.stream, c.elem_faces, ops, half,
 			                   a.out, c.E);
 			return hipGetLastError();
 		}
