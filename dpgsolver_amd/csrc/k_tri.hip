@@ -1032,8 +1032,8 @@ __device__ inline void mix_faces(const MixArgsT<T>& a, int start, int count, int
 	const int q = j;
 	T g[kNV];
 	if (valid && j < NF) {
-		const T Jf = tsqrt(nj0 * nj0 + nj1 * nj1), Jfi = trcp(Jf);
-		const T nu[2] = { nj0 * Jfi, nj1 * Jfi };
+		const T Jf = sqrt(nj0 * nj0 + nj1 * nj1);
+		const T nu[2] = { nj0 / Jf, nj1 / Jf };
 		T sL[kNV], sR[kNV], nnf[kNV];
 		side_at_point<NF>(o, f.kL, f.NL, q, F, sL);
 		if (inter) side_at_point<NF>(o, f.kR, f.NR, f.rev ? NF - 1 - q : q, F + kNV * NF, sR);
@@ -1153,8 +1153,8 @@ __device__ inline void mix_faces_ns(const MixArgsT<T>& a, int start, int count, 
 		if (inter) {
 			side_at_point<NF>(o, f.kR, f.NR, qr, YL + kNV * NF, sR);
 		} else {   // the boundary state (Riemann or a no-slip wall) at this point
-			const T Jfi = trcp(tsqrt(nj0 * nj0 + nj1 * nj1));
-			const T nu[2] = { nj0 * Jfi, nj1 * Jfi };
+			const T Jf = sqrt(nj0 * nj0 + nj1 * nj1);
+			const T nu[2] = { nj0 / Jf, nj1 / Jf };
 			double xy[2] = { 0.0, 0.0 };
 			if (f.bc == DGX_BC_NOSLIP_ROTATING) {
 				xy[0] = a.wxy[((size_t)fi * kHpMaxN + q) * 2];
@@ -1209,8 +1209,8 @@ __device__ inline void mix_faces_ns(const MixArgsT<T>& a, int start, int count, 
 	wave_sync();
 	T fq[kNV];
 	if (point) {   // the flux at this face point: inviscid first, then each side's face gradient P h and viscous flux
-		const T Jf = tsqrt(nj0 * nj0 + nj1 * nj1), Jfi = trcp(Jf);
-		const T nu[2] = { nj0 * Jfi, nj1 * Jfi };
+		const T Jf = sqrt(nj0 * nj0 + nj1 * nj1);
+		const T nu[2] = { nj0 / Jf, nj1 / Jf };
 		T nnf[kNV], fvL[K8], fvR[K8];
 		if constexpr (FLUX == DGX_FLUX_LF) numflux_lf<T, 2>(sL, sR, nu, nnf);
 		else numflux_roe<T, 2>(sL, sR, nu, nnf);
