@@ -287,8 +287,8 @@ dgx_status dgx_graph_sync(dgx_graph* g, double* max_abs_r);
 dgx_status dgx_graph_destroy(dgx_graph* g);
 /* Launch shape of the residual kernels.  The grid is either one workgroup per element block (the default,
  * grid 0) or persistent: `grid` workgroups, each XCD's share striding over that XCD's contiguous range of
- * element blocks with the reference-element operators staged in LDS once.  kind: DGX_GRAPH_RHS_FP64, _FP32,
- * _MIXED, or DGX_TUNE_RHS_MINV (the M^-1 R launch of the explicit step).  The persistent kernel is a separate
+ * element blocks.  kind: DGX_GRAPH_RHS_FP64, _FP32, _MIXED, or DGX_TUNE_RHS_MINV (the M^-1 R launch of
+ * dgx_compute_rhs_explicit; dgx_ssp_rk3_step has stage kernels of its own).  The persistent kernel is a separate
  * compilation of the same code; its results agree with the default kernel's to rounding (the compiler may
  * pair multiplies and adds into FMAs differently), not bit for bit. */
 enum { DGX_TUNE_RHS_MINV = 3 };

@@ -47,3 +47,32 @@ def test_limited_step_matches_oracle(d, p, n):
         ctx.ssp_rk3_step(low.data_ptr(), 0.0, positivity=True)
     assert e.value.code == -4
     ctx.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_step_does_not_depend_on_the_residual_grid(graph):
+    """A persistent grid for the M^-1 R kernel leaves the stage kernels of the step alone: the same step bit for bit."""
+    from dpgsolver_amd import _lib
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    mesh = M.config2_mesh(24, 3)
+    u = M.config2_state(mesh)
+    ctx = _lib.Context(2, 3, M.PDE_EULER, M.FLUX_ROE)
+    ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+    ctx.upload_mesh(mesh.xyz, mesh.faces)
+    out = []
+    for grid in (0, 256):
+        ctx.set_rhs_grid(_lib.TUNE_RHS_MINV, grid)
+        ud = torch.from_numpy(u).to("cuda:0")
+        if graph:
+            g = ctx.graph_rk3(ud.data_ptr(), 1e-3, positivity=True)
+            g.launch(2)
+            mx = g.sync()
+            g.close()
+        else:
+            for _ in range(2):
+                mx = ctx.ssp_rk3_step(ud.data_ptr(), 1e-3, positivity=True)
+        out.append((ud, mx))
+    assert torch.equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+    ctx.close()
