@@ -588,7 +588,8 @@ struct dgx_mlp {
 	int step = 0;
 	int cap = 0;
 	float *h1 = nullptr, *h2 = nullptr, *o = nullptr, *go = nullptr, *gh2 = nullptr, *gh1 = nullptr;
-	float* gpart = nullptr;   // planes of the product cut along K (see k_gemm_bf16)
+	float* gpart = nullptr;   // planes of the product cut along K (see k_gemm_bf16), backward pass only
+	int gcap = 0;             // samples that gpart holds
 	double* lpart = nullptr;
 	double* lall = nullptr;   // per-sample losses of a whole training set
 	long long lall_cap = 0;
@@ -609,7 +610,7 @@ static void mlp_free_work(dgx_mlp* m)
 	m->lall_cap = 0;
 	m->h1 = m->h2 = m->o = m->go = m->gh2 = m->gh1 = m->gpart = nullptr;
 	m->lpart = nullptr;
-	m->cap = 0;
+	m->cap = m->gcap = 0;
 }
 
 static hipError_t mlp_reserve(dgx_mlp* m, int B)
@@ -623,7 +624,6 @@ static hipError_t mlp_reserve(dgx_mlp* m, int B)
 	DGX_HIP_CHECK(hipMalloc(&m->gh2, sizeof(float) * (size_t)B * m->nhid));
 	DGX_HIP_CHECK(hipMalloc(&m->gh1, sizeof(float) * (size_t)B * m->nhid));
 	DGX_HIP_CHECK(hipMalloc(&m->lpart, sizeof(double) * (size_t)B));
-	DGX_HIP_CHECK(hipMalloc(&m->gpart, sizeof(float) * (size_t)B * m->nhid * kSplits));
 	m->cap = B;
 	return hipSuccess;
 }
@@ -652,6 +652,13 @@ static hipError_t mlp_backward(dgx_mlp* m, const float* X, int B)
 {
 	const float *W2 = m->wb + m->off[2], *W3 = m->wb + m->off[4];
 	const int nf = m->nf, nh = m->nhid, no = m->nout;
+	if (B > m->gcap) {   // inference, over as many samples as there are elements, does without these planes
+		if (m->gpart) (void)hipFree(m->gpart);
+		m->gpart = nullptr;
+		m->gcap = 0;
+		DGX_HIP_CHECK(hipMalloc(&m->gpart, sizeof(float) * (size_t)B * nh * kSplits));
+		m->gcap = B;
+	}
 	// the sum over the outputs is the one long K range: cut over kSplits workgroups a tile
 	GemmJob gh = gemm_job(m->go, no, 1, W3, nh, 0, m->gpart, nh, B, nh, no);
 	gh.splits = kSplits;

@@ -34,3 +34,26 @@ def test_loss_gradient_at_odd_sizes(nb, Np, kind, rank, hidden, B):
     for a, b in zip(offs, offs[1:] + [n]):
         assert np.linalg.norm(g[a:b] - gref[a:b]) <= 5e-3 * np.linalg.norm(gref[a:b]) + 1e-12
     m.close()
+
+
+def test_inference_takes_no_training_planes():
+    """dgx_mlp_predict over many samples holds three activations, their gradients and the losses, not the split planes of
+    the backward pass (4 B hidden floats more); training after it still finds them."""
+    from dpgsolver_amd import _lib
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    B, hidden = 100000, 512
+    m = _lib.MLP(36, 9, hidden=hidden, rank=4, seed=7, kind=1)
+    X = torch.zeros((B, m.nf), dtype=torch.float32, device="cuda:0")
+    out = torch.empty((B, m.nout), dtype=torch.float32, device="cuda:0")
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    m.predict(X.data_ptr(), B, out.data_ptr())
+    torch.cuda.synchronize()
+    took = free0 - torch.cuda.mem_get_info()[0]
+    need = 4 * B * (4 * hidden + 2 * m.nout) + 8 * B
+    assert took <= need + 64 * 2 ** 20, (took, need)      # (the planes alone: 819 MB)
+    A = torch.eye(36, dtype=torch.float64, device="cuda:0").repeat(40, 1, 1)
+    assert np.isfinite(m.train(X.data_ptr(), None, A.data_ptr(), 40, epochs=1, batch=16, lr=1e-4))
+    m.close()
