@@ -93,6 +93,15 @@ __device__ inline int face_vol_node(int lf, int i)
 	return a + N * (b + N * fix);
 }
 
+// acc + m x with one rounding, written out: left to the compiler, which of a two-term sum's products it rounds first changes
+// with the code around it
+__device__ inline float mul_add(float m, float x, float acc) { return __builtin_fmaf(m, x, acc); }
+__device__ inline double mul_add(double m, double x, double acc) { return __builtin_fma(m, x, acc); }
+template <typename R>
+__device__ inline Dual mul_add(R m, Dual x, Dual acc) { return acc + m * x; }
+template <typename R>
+__device__ inline Dual32 mul_add(R m, Dual32 x, Dual32 acc) { return acc + m * x; }
+
 // The sweeps are always inlined: as functions they take the operators by vector loads and hold a whole call's registers
 // (HEX linear operator p = 4 28^3 914 -> 387 us, p = 2 373 -> 117, p = 1 118 -> 52).
 //
@@ -126,7 +135,7 @@ __device__ __forceinline__ void sweep_inplace(S* buf, const R* M, int dir, int t
 			for (int q = 0; q < N; ++q) {
 				S acc = M[q * N] * in[k][0];
 #pragma unroll
-				for (int j = 1; j < N; ++j) acc += M[q * N + j] * in[k][j];
+				for (int j = 1; j < N; ++j) acc = N == 2 ? mul_add(M[q * N + j], in[k][j], acc) : acc + M[q * N + j] * in[k][j];
 				buf[base[k] + q * Sd] = acc;
 			}
 		}
@@ -172,7 +181,7 @@ __device__ __forceinline__ void sweep_inplace2(S* buf, const R* M, int dir, int 
 			for (int q = 0; q < N; ++q) {
 				S acc = M[q * N] * in[k][0];
 #pragma unroll
-				for (int j = 1; j < N; ++j) acc += M[q * N + j] * in[k][j];
+				for (int j = 1; j < N; ++j) acc = N == 2 ? mul_add(M[q * N + j], in[k][j], acc) : acc + M[q * N + j] * in[k][j];
 				buf[base[k] + q * Sd] = acc;
 			}
 		}
@@ -236,7 +245,7 @@ __device__ __forceinline__ void sweep_to(const S* src, S* dst, const R* M, int d
 			for (int q = 0; q < N; ++q) {
 				S acc = M[q * N] * in[0];
 #pragma unroll
-				for (int j = 1; j < N; ++j) acc += M[q * N + j] * in[j];
+				for (int j = 1; j < N; ++j) acc = N == 2 ? mul_add(M[q * N + j], in[j], acc) : acc + M[q * N + j] * in[j];
 				if (ACC) dst[base + q * Sd] += acc;
 				else dst[base + q * Sd] = acc;
 			}
