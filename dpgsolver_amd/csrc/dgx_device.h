@@ -66,11 +66,12 @@ __device__ inline double rv(Dual a) { return a.v; }
 __device__ inline float rv(Dual32 a) { return a.v; }
 
 // FP64 reciprocal and square root: the hardware's first approximation (2^-24) and two Newton steps, which leave the
-// rounding of the last multiply-add (a million values in 2^-900 .. 2^900: none differs from the IEEE result).  The IEEE
-// sequences of 1.0 / a and sqrt(a) also scale for residuals that underflow, 11 and 18 instructions for these 6 and 11, and
+// rounding of the last multiply-add.  The IEEE sequences of 1.0 / a and sqrt(a) also scale for residuals that underflow, 11
+// and 18 instructions for these 6 and 11, and
 // the kernels with FP64 pointwise fluxes are bound by instruction issue.  With the Lax-Friedrichs flux below on unnormalised
 // normals: HEX p = 4, 64^3 mixed 1723 -> 1612 us, 32^3 FP64 286 -> 279 us, Navier-Stokes 448 x 448 242 -> 238 us.
-// Zero, infinity and NaN come out as in the IEEE sequences.
+// Zero, infinity and NaN come out as in the IEEE sequences.  Subnormal values do not: their reciprocals (2^1022 and beyond)
+// may come out as NaN.
 __device__ inline double trcp(double a)
 {
 	double r = __builtin_amdgcn_rcp(a);

@@ -933,7 +933,7 @@ struct PrecondBlockSGS : Precond {
 	bool reducible(const Ctx& c) const override { return !fp32 && (int)c.color_off.size() == 3 && !c.self_neighbour; }
 	static size_t count(const Ctx& c, int k) { return (size_t)(c.color_off[k + 1] - c.color_off[k]); }
 	static int rows(const Ctx& c) { return c.nv * (4 * c.N - 4); }
-	// the packed kernels' sizes: nv = 4, N <= 5 (the largest order that the in-LDS inverse takes)
+	// the packed kernels' sizes: nv = 4, N <= 5 (the largest order that the batched inverse takes)
 	bool faces_only(const Ctx& c) const { return reducible(c) && c.d == 2 && !full(c) && c.nv == 4 && c.N <= 5; }
 	size_t reduced_size(const Ctx& c) const override { return count(c, 1) * (faces_only(c) ? rows(c) : c.Np * c.nv); }
 	hipError_t face_rows(Ctx& c, const double* src, double* dst, bool expand)
@@ -1266,13 +1266,13 @@ struct Gmres {
 using dgx::Ctx;
 
 // 3-D (HEX Euler): the FP64 J v, and no preconditioner, block-Jacobi with blocks the batched LU takes
-// (nb = 5 (p + 1)^3 <= 143: p <= 2), or block SGS with blocks the in-LDS inverse and the sweep take (p <= 2)
+// (nb = 5 (p + 1)^3 <= 143: p <= 2), or block SGS with blocks the batched inverse and the sweep take (p <= 2)
 static bool implicit_3d_ok(const Ctx& c, int precond, int jvp_fp32)
 {
 	if (c.d != 3) return true;
 	if (jvp_fp32) return false;
 	if (precond == DGX_PC_NONE) return true;
-	if (precond == DGX_PC_BLOCK_SGS || precond == DGX_PC_BLOCK_SGS32)   // in-LDS inverses (nb <= 142: p <= 2)
+	if (precond == DGX_PC_BLOCK_SGS || precond == DGX_PC_BLOCK_SGS32)   // batched inverses (nb <= 142: p <= 2)
 		return c.Np * c.nv <= dgx::kMaxInvBlock && 6 * c.nv * c.N * c.N <= dgx::kMaxSgsFace;
 	return precond == DGX_PC_BLOCK_JACOBI && c.Np * c.nv <= dgx::kMaxLuBlock;
 }

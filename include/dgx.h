@@ -354,7 +354,7 @@ dgx_status dgx_newton_operator(dgx_ctx* ctx, const double* u, const double* mass
 dgx_status dgx_block_lu_factor(dgx_ctx* ctx, double* blocks, int* piv, int E, int nb);
 /* x <- A_e^{-1} x for every element block (x: E*nb). */
 dgx_status dgx_block_lu_solve(dgx_ctx* ctx, const double* lu, const int* piv, double* x, int E, int nb);
-/* In-place inverse of E blocks of size nb <= 142 (Gauss-Jordan, partial pivoting, a block in LDS), stored transposed:
+/* In-place inverse of E blocks of size nb <= 142 (Gauss-Jordan, partial pivoting), stored transposed:
  * blocks[e][j * nb + i] = (A_e^-1)[i][j].  The block-Jacobi preconditioner applies it as one mat-vec. */
 dgx_status dgx_block_inverse(dgx_ctx* ctx, double* blocks, int E, int nb);
 /* y_e = A_e^-1 x_e from the transposed inverses of dgx_block_inverse (x, y: E*nb, distinct). */
@@ -371,7 +371,8 @@ dgx_status dgx_block_inv_apply(dgx_ctx* ctx, const double* inv, const double* x,
  * PETSc ILU(1) with RCM ordering (external/petsc/options_files/petsc_options_gmres_default.txt:6-8), which
  * factors the assembled matrix sequentially.  DGX_PC_BLOCK_SGS32: the same sweeps with the inverse diagonal
  * blocks and the face blocks stored in FP32 (half the bytes the sweeps read; products and sums in FP64, the
- * vectors FP64).  DGX_PC_LEARNED: the MLP below. */
+ * vectors FP64).  On meshes of two colours without self-neighbouring elements DGX_PC_BLOCK_SGS builds GMRES on
+ * one colour alone, which SGS32 does not, and is the faster of the two there.  DGX_PC_LEARNED: the MLP below. */
 enum { DGX_PC_NONE = 0, DGX_PC_BLOCK_JACOBI = 1, DGX_PC_LEARNED = 2, DGX_PC_BLOCK_SGS = 3, DGX_PC_BLOCK_SGS32 = 4 };
 /* z = P^-1 v for one preconditioner set up at state u with the pseudo-time scale inv_dt (E doubles, as
  * dgx_cfl_dt writes it): the operator that dgx_solve_implicit applies inside GMRES, exposed for callers that
@@ -401,7 +402,10 @@ typedef struct dgx_implicit_params {
 	int jvp_fp32;         /* 1: the GMRES operator dR/du v - M v / dt in FP32 dual numbers (FP64 vectors; Euler:
 	                         FP32 geometry and operators, Navier-Stokes: FP64 ones converted as they are read): the
 	                         inner defect-correction product; the FP64 residual of
-	                         each Newton step still decides convergence.  0: FP64 (no counterpart: the reference
+	                         each Newton step still decides convergence.  Where
+	                         DGX_PC_BLOCK_SGS solves on a two-coloured mesh, GMRES
+	                         takes its products from the assembled FP64 blocks and
+	                         this product only at restarts.  0: FP64 (no counterpart: the reference
 	                         assembles the FP64 Jacobian) */
 } dgx_implicit_params;
 typedef struct dgx_implicit_stats {

@@ -13,7 +13,7 @@
   than block-Jacobi.
 * The 3-D face blocks, the block-sparse export and the SGS sweeps are checked against the oracle and numpy with
   the 2-D ones (test_gpu_solvers.py, the hex_* cases).
-* 3-D paths with no counterpart here (FP32 J v, blocks beyond the in-LDS inverse and LU: p >= 3) return
+* 3-D paths with no counterpart here (FP32 J v, blocks beyond the batched inverse and LU: p >= 3) return
   DGX_ERR_UNSUPPORTED.
 """
 import numpy as np
@@ -152,7 +152,7 @@ def test_steady_box_3d_newton_gmres(dev):
 
 
 def test_steady_box_3d_p2_block_jacobi_and_sgs(dev):
-    """p = 2 (nb = 135): block-Jacobi and block SGS over in-LDS inverses of 146 KB blocks (270 face dofs per
+    """p = 2 (nb = 135): block-Jacobi and block SGS over batched inverses of 146 KB blocks (270 face dofs per
     element in the SGS sweep)."""
     from dpgsolver_amd import _lib
 
@@ -182,7 +182,7 @@ def test_3d_unsupported_paths_are_refused(dev):
     with pytest.raises(_lib.DgxError, match="UNSUPPORTED"):
         ctx.solve_implicit(ud.data_ptr(), precond=_lib.PC_BLOCK_JACOBI, jvp_fp32=True)
     ctx.close()
-    mesh3, u3 = _curved(3, 2, 3)    # nb = 320: more than the batched LU and the in-LDS inverse take
+    mesh3, u3 = _curved(3, 2, 3)    # nb = 320: more than the batched LU and inverse take
     ctx = _ctx(mesh3, M.FLUX_ROE)
     ud = torch.from_numpy(u3).to(dev)
     for pc in (_lib.PC_BLOCK_JACOBI, _lib.PC_BLOCK_SGS, _lib.PC_BLOCK_SGS32):

@@ -116,7 +116,7 @@ def _jac_cases():
     pert = 0.02 * np.sin(3 * x[..., 0]) * np.cos(2 * x[..., 1]) * np.cos(x[..., 2])
     u = M.pack_state(M.prim_to_cons(prim[None, None, :] * (1.0 + np.stack([pert, pert, -pert, pert, 0.5 * pert], -1)), 3))
     out.append(("hex_box_lf_p1", m, M.FLUX_LF, prim, u))
-    # the largest blocks of the in-LDS inverse: QUAD Euler p = 4 (nb = 100) and HEX p = 2 (nb = 135, 270 face dofs)
+    # the largest blocks of the batched inverse: QUAD Euler p = 4 (nb = 100) and HEX p = 2 (nb = 135, 270 face dofs)
     m = M.structured_tp_mesh(2, 4, (3, 3), (0, 0), (1, 1), (True, True),
                              rotate=np.random.default_rng(6).integers(0, 4, 9))
     u = M.pack_state(M.prim_to_cons(M.smooth_state_3d(M.nodes_xyz(m)), 2))
@@ -387,7 +387,7 @@ def test_block_lu_solve_matches_numpy(dev):
     with pytest.raises(_lib.DgxError):
         ctx.block_lu_factor(Ad.data_ptr(), piv.data_ptr(), 1, 144)
     # the explicit (transposed) inverse used by the block-Jacobi and block SGS preconditioners, with pivoting
-    # exercised; nb = 135 and 142 take more than 64 KB of LDS per block
+    # exercised; nb = 135 and 142 take four wavefronts and nine tiles of 16 rows per block
     for E, nb in ((37, 64), (9, 135), (4, 142)):
         A = rng.standard_normal((E, nb, nb)) / np.sqrt(nb) + 4 * np.eye(nb)
         x = rng.standard_normal((E, nb))
