@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(128) k_ns_gv(NsArgs<S> a)
 // them; k_ns_add then lifts the neighbours' halves onto the face nodes.  A boundary face has no other half.
 // Bound by memory: per element of QUAD p = 3 FP64 state, geometry, residual and halves are 2.2 KB here and 1.1 KB in
 // k_ns_add, where the gradient traces (1 KB written, 2 KB read back) made it 6.5 KB; the volume gradient is computed
-// once instead of twice.  448 x 448, Roe, FP64: 306 -> 242 us (222 here: the FP64 pipe takes 138, LDS 122 of them).
+// once instead of twice.  448 x 448, Roe, FP64: 306 -> 238 us (209 here: the FP64 pipe takes 138, LDS 122 of them).
 // LDS regions change hands: the face traces (own and neighbour) become the face products in place, the volume gradient
 // becomes the weighted fluxes, the GLL state becomes the face fluxes.
 // The mixed form (PERT) keeps the halves in FP64, as its face fluxes are: rounded to FP32 on their way they added to the
@@ -894,7 +894,7 @@ __global__ void __launch_bounds__(128) k_rhs_ns(NsArgs<S> a)
 
 // phase 0: the whole residual; 1: the gradient traces only; 2: the residual only (variable-order meshes run the
 // face kernel between orders in between).  The residual needs no other element's gradient traces in phase 0, so it takes
-// k_ns_own and k_ns_add there (242 us against 306 at 448 x 448, p = 3, FP64); the dual numbers of the linearisation keep
+// k_ns_own and k_ns_add there (238 us against 306 at 448 x 448, p = 3, FP64); the dual numbers of the linearisation keep
 // the gradient-trace kernels, whose traces every block column reads.
 template <typename S, int N, bool PERT, int MODE>
 hipError_t run_ns(Ctx& c, const NsArgs<S>& a, int phase)
